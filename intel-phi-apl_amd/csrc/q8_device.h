@@ -278,6 +278,20 @@ struct q8_gemm_round {
 int q8_launch_gemm_round(q8_stream_t stream, int n, const void *const *w, const long *rows, long cols, const float *x, long x_stride, long t,
                          float *const *y, float *part, long part_cap, q8_gemm_opts o, float *pair_y = nullptr);
 long q8_gemm_round_part_floats(int n, const long *rows, long cols, long t, q8_gemm_opts o);
+/* The K split of a rows x cols matrix: ks splits of cps ranges of Q8_SPLIT_PAIRS pairs of blocks (the
+ * last may hold fewer), a function of the shape alone (o.ks > 0 forces it). */
+#define Q8_SPLIT_PAIRS 2
+void q8_gemm_split(long rows, long cols, q8_gemm_opts o, int *ks, int *cps);
+/* More than 64 tokens as one launch (q8_tile.hip): whether it takes n products sharing x (pair: the
+ * fused pair, n == 2 of one shape) and is the faster route, from their sizes alone. Then the limb
+ * image of x (of its RMS norm when nw != NULL) at img, q8_ximage_bytes(t, cols) bytes, below 2^31, 16-byte aligned,
+ * and the launch: y[i] = X w[i]^T (plus res when given, n == 1), or pair_y = SiLU(G) * U. The bits
+ * are those of the 64-token launches. */
+long q8_ximage_bytes(long t, long cols);
+bool q8_tile_takes(int n, const long *rows, long cols, long t, bool pair);
+void q8_launch_ximage(q8_stream_t stream, const float *x, long x_stride, long t, long cols, const float *nw, float eps, void *img);
+void q8_launch_tile(q8_stream_t stream, int n, const void *const *w, const long *rows, long cols, long t, const void *img, float *const *y, const float *res,
+                    float *pair_y, q8_gemm_opts o);
 /* The floor of the x-resident product at 5 <= t <= 16 tokens: its loads on its grid (the plan for
  * these options), no arithmetic, a checksum added to sink[0]; -1 when the plan is not the
  * x-resident kernel. */

@@ -801,7 +801,7 @@ struct gemm_cfg {
 
 /* the x-resident kernel for one token tile: 2-pair ranges, 16 or 12 waves, segments of 8 ranges
  * (x limbs 96 KiB and scales 13-17 KiB of LDS: one workgroup a CU) */
-#define XRES_KP 2
+#define XRES_KP Q8_SPLIT_PAIRS
 #define XRES_SC 8
 
 /* every configuration streams ranges of the same KP pairs, so a K split of cps ranges covers the
@@ -905,6 +905,8 @@ static gemm_plan plan_of(long rows, long cols, long t, q8_gemm_opts o)
     split_of(rows, cols, nw, o.ks, &p.ks, &p.cps);
     return p;
 }
+
+void q8_gemm_split(long rows, long cols, q8_gemm_opts o, int *ks, int *cps) { split_of(rows, cols, nw_of(rows, cols, o.ks), o.ks, ks, cps); }
 
 long q8_gemm_part_floats(long rows, long cols, long t, q8_gemm_opts o)
 {

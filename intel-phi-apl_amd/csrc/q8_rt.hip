@@ -116,6 +116,8 @@ struct ctx {
     /* a matrix-core round's partials, every product's */
     float *rpart = nullptr;
     size_t rpart_cap = 0;
+    /* the limb image of a long prompt's x (q8_tile.hip), TILE_IMG_BYTES */
+    void *ximg = nullptr;
     /* the device address of `scratch` on this runtime's GPU (rt_gemm_dev_noalloc's partials) */
     float *noalloc_part = nullptr;
     /* the greedy next token's candidates */
@@ -144,6 +146,15 @@ struct ctx {
 };
 
 constexpr size_t KT_MAX = 16384;
+
+/* The workspace of a long prompt's limb image: 64 MiB hold 910 tokens of 12288 columns, 2730 of 4096;
+ * longer prompts run in chunks of that many, each reading the weights again, which a chunk of
+ * hundreds of tokens hides behind its arithmetic. Of one size, so that a graph may record any shape
+ * once one long product has run. */
+constexpr long TILE_IMG_BYTES = 64L << 20;
+/* Rounds run as one launch from 81 tokens, single products and the fused pair from 65: the tests
+ * hold the rounds of 65 to 70 tokens to the 64-token round kernels by name. */
+constexpr long TILE_ROUND_MIN = 81;
 
 /* The runtimes alive, in the order rt_init set them up; rt_q8_row takes no struct rt
  * (src/card/rt.h:85) and uses the last of them. */
@@ -303,12 +314,67 @@ void reserve_gemm(ctx *c, long rows, long cols, long t)
         fail("the matrix-core product", "its K-split partials exceed the workspace (a planning error)");
 }
 
+/* the partials of a round's 64-token launches */
+float *reserve_round(ctx *c, int n, const long *rows, long cols, long t)
+{
+    return reserve_rpart(c, (size_t)q8_gemm_round_part_floats(n, rows, cols, t < 64 ? t : 64, c->gemm_opts));
+}
+
+/* the fused pair's two products (g) and their partials (rp) on the 64-token launches */
+void reserve_pair(ctx *c, long rows, long cols, long t, float **g, float **rp)
+{
+    const long r2[2] = {rows, rows};
+    *g = reserve_scratch(c, (size_t)(2 * rows * t));
+    *rp = reserve_round(c, 2, r2, cols, t);
+}
+
 /* Whether a product of t tokens runs on the matrix cores (every 64-token launch of it, the last
  * one too, however few tokens it holds, so that a token's bits do not depend on t), else on the
  * decode kernels, which take at most 4 tokens a launch. */
 bool on_matrix_cores(long t) { return t >= 5; }
 
-/* Y = X W^T for t >= 5 tokens on the matrix cores, 64 at a time; res != NULL: Y = res + X W^T (res
+/* Whether these products of more than 64 tokens run as one launch (q8_tile.hip), and their workspace
+ * is there: the library's, allocated at its first use outside a recording, or part, a caller's of
+ * Q8_GEMM_PART_MAX floats. Where not, the 64-token launches give the same bits. */
+bool tile_ready(ctx *c, int n, const long *rows, long cols, long t, bool pair, const float *part)
+{
+    if (!q8_tile_takes(n, rows, cols, t, pair) || q8_ximage_bytes(128, cols) > (part ? Q8_GEMM_PART_MAX * (long)sizeof(float) : TILE_IMG_BYTES))
+        return false;
+    if (part || c->ximg)
+        return true;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    HIPCHECK(hipStreamIsCapturing(c->stream, &st));
+    if (st != hipStreamCaptureStatusNone)
+        return false;
+    if (hipMalloc(&c->ximg, (size_t)TILE_IMG_BYTES) != hipSuccess) {
+        (void)hipGetLastError();
+        c->ximg = nullptr;
+        return false;
+    }
+    return true;
+}
+
+/* The products, after tile_ready: y[i] = X w[i]^T (of RMS(X) when nw != NULL; plus res when given,
+ * one product), or pair_y = SiLU(X w[0]^T) * (X w[1]^T); in chunks of as many tokens as the image
+ * holds, as equal as whole 128-token groups allow. */
+void tile_run(ctx *c, int n, const void *const *w, const long *rows, long cols, const float *x, long xs, long t, float *const *y, const float *res,
+              float *pair_y, const float *nw, float eps, float *part)
+{
+    const q8_stream_t s = (q8_stream_t)c->stream;
+    void *img = part ? (void *)part : c->ximg;
+    const long most = (part ? Q8_GEMM_PART_MAX * (long)sizeof(float) : TILE_IMG_BYTES) / q8_ximage_bytes(128, cols) * 128;
+    const long chunks = (t + most - 1) / most, per = ((t + chunks - 1) / chunks + 127) / 128 * 128;
+    for (long k = 0; k < t; k += per) {
+        const long tk = t - k < per ? t - k : per;
+        float *yk[RT_BATCH] = {};
+        for (int i = 0; i < n && !pair_y; i++)
+            yk[i] = y[i] + k * rows[i];
+        q8_launch_ximage(s, x + k * xs, xs, tk, cols, nw, eps, img);
+        q8_launch_tile(s, n, w, rows, cols, tk, img, yk, res ? res + k * rows[0] : nullptr, pair_y ? pair_y + k * rows[0] : nullptr, c->gemm_opts);
+    }
+}
+
+/* Y = X W^T for t >= 5 tokens on the matrix cores, 64 at a time (or as one launch of more); res != NULL: Y = res + X W^T (res
  * may be Y), added in the matrix-core product's store or partial sum. part != NULL: the K-split
  * partials go there (at most Q8_GEMM_PART_MAX floats) instead of the runtime's workspace, and
  * nothing is allocated. */
@@ -316,6 +382,12 @@ void gemm_tokens(ctx *c, const void *w, long rows, long cols, const float *x, lo
                  float *part = nullptr)
 {
     const q8_stream_t s = (q8_stream_t)c->stream;
+    if (tile_ready(c, 1, &rows, cols, t, false, part)) {
+        if (!part)
+            reserve_gemm(c, rows, cols, 64); /* as the 64-token launches: a later recording may count on it */
+        tile_run(c, 1, &w, &rows, cols, x, xs, t, &y, res, nullptr, nullptr, 0.0f, part);
+        return;
+    }
     for (long k = 0; k < t; k += 64) {
         const long n = t - k < 64 ? t - k : 64;
         if (part) {
@@ -367,14 +439,18 @@ void product(ctx *c, const void *w0, const void *w1, long rows, long cols, const
     } else if (!w1) {
         gemm_tokens(c, w0, rows, cols, x, xs, t, y, nullptr, part);
     } else {
-        float *g = reserve_scratch(c, (size_t)(2 * rows * t));
+        float *g, *rp;
+        reserve_pair(c, rows, cols, t, &g, &rp);
         /* 64 tokens at a time, the gate and the up product as one round, their sums and the SwiGLU
          * in one launch: the same sums and SwiGLU as apart (below, where the round is refused) */
         const void *w2[2] = {w0, w1};
         const long r2[2] = {rows, rows};
-        const long t0 = t < 64 ? t : 64;
-        float *rp = reserve_rpart(c, (size_t)q8_gemm_round_part_floats(2, r2, cols, t0, c->gemm_opts));
         bool pair_done = true;
+        if (tile_ready(c, 2, r2, cols, t, true, nullptr)) {
+            tile_run(c, 2, w2, r2, cols, x, xs, t, nullptr, nullptr, y, nullptr, 0.0f, nullptr);
+            launched("the fused pair");
+            return;
+        }
         for (long k = 0; k < t && pair_done; k += 64) {
             const long tk = t - k < 64 ? t - k : 64;
             float *y2[2] = {g, g + rows * tk};
@@ -431,6 +507,22 @@ void product_epi(ctx *c, const void *w0, const void *w1, long rows, long cols, c
     }
     if (e.nw) {
         float *xn = reserve_epi(c, (size_t)(t * cols));
+        const void *w2[2] = {w0, w1};
+        const long r2[2] = {rows, rows};
+        if (!c->exact && !apart && tile_ready(c, w1 ? 2 : 1, r2, cols, t, w1 != nullptr, nullptr)) {
+            /* the norm in the limb image: the same sum and the same xn as apart. The workspaces as
+             * product() reserves them: a later recording of fewer tokens may count on them */
+            if (w1) {
+                float *g, *rp;
+                reserve_pair(c, rows, cols, t, &g, &rp);
+            } else {
+                reserve_gemm(c, rows, cols, 64);
+            }
+            kt_begin(c, w1 ? RT_K_GEMM_PAIR : RT_K_GEMM, rows, cols, t);
+            tile_run(c, w1 ? 2 : 1, w2, r2, cols, x, xs, t, &y, nullptr, w1 ? y : nullptr, e.nw, e.eps, nullptr);
+            launched("the product on the norm");
+            return;
+        }
         q8_launch_rmsnorm(s, x, xs, t, cols, e.nw, e.eps, xn);
         launched("the norm");
         product(c, w0, w1, rows, cols, xn, cols, t, y);
@@ -469,8 +561,13 @@ bool round_launch(ctx *c, int n, const void *const *w, const long *rows, long co
         rc = q8_launch_gemv_round((q8_stream_t)c->stream, n, w, rows, cols, x, xs, t, y);
     } else {
         /* 64 tokens at a time (a token's bits do not depend on t) */
-        float *rp = reserve_rpart(c, (size_t)q8_gemm_round_part_floats(n, rows, cols, t < 64 ? t : 64, c->gemm_opts));
+        float *rp = reserve_round(c, n, rows, cols, t);
         rc = 0;
+        if (t >= TILE_ROUND_MIN && tile_ready(c, n, rows, cols, t, false, nullptr)) {
+            tile_run(c, n, w, rows, cols, x, xs, t, y, nullptr, nullptr, nullptr, 0.0f, nullptr);
+            launched("the round");
+            return true;
+        }
         for (long k = 0; k < t && rc == 0; k += 64) {
             const long tk = t - k < 64 ? t - k : 64;
             float *yk[RT_BATCH];
@@ -695,6 +792,8 @@ void rt_fini(struct rt *R)
         HIPCHECK(hipFree(c->epi));
     if (c->rpart)
         HIPCHECK(hipFree(c->rpart));
+    if (c->ximg)
+        HIPCHECK(hipFree(c->ximg));
     for (void *p : c->retired)
         HIPCHECK(hipFree(p));
     for (auto &e : c->kt_events)
@@ -1051,6 +1150,16 @@ void rt_gemv_round_norm_dev(struct rt *R, int n, const void *const *w, const lon
             kt_cancel(c);
     }
     float *xn = reserve_epi(c, (size_t)(t * cols));
+    if (!c->exact && n > 1 && !c->epi_apart && t >= TILE_ROUND_MIN && tile_ready(c, n, rows, cols, t, false, nullptr)) {
+        reserve_round(c, n, rows, cols, t);
+        long total = 0;
+        for (int i = 0; i < n; i++)
+            total += rows[i];
+        kt_begin(c, RT_K_ROUND, total, cols, t);
+        tile_run(c, n, w, rows, cols, x, x_stride, t, y, nullptr, nullptr, nw, eps, nullptr);
+        launched("the round on the norm");
+        return;
+    }
     q8_launch_rmsnorm(s, x, x_stride, t, cols, nw, eps, xn);
     launched("the norm");
     if (!c->exact && n > 1 && round_launch(c, n, w, rows, cols, xn, cols, t, y))

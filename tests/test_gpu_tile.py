@@ -1,0 +1,212 @@
+"""Products of more than 64 tokens as one launch (csrc/q8_tile.hip) against the 64-token launches,
+bit for bit: the same sums in the same order, at every tile configuration, partial tiles of rows and
+tokens, odd block counts (half a last pair, 2-byte aligned scales), forced K splits (one, and a
+shorter last one), the residual, the norm, the fused pair, rounds, non-finite x and scales, chunks of
+the limb image, and under graph capture."""
+import ctypes as c
+
+import numpy as np
+import pytest
+
+import synth
+from parity import assert_parity
+
+pytestmark = pytest.mark.gpu
+
+P = c.c_void_p
+
+
+def kernels(rt, fn):
+    """The names of the first kernels of the products fn launches (the runtime's records)."""
+    n = 256
+    rt.lib.rt_ktime(rt.R, 1)
+    fn()
+    arrs = [np.zeros(n, np.int32), np.zeros(n, np.int64), np.zeros(n, np.int64), np.zeros(n, np.int64), np.zeros(n, np.float32)]
+    names, grid = c.create_string_buffer(64 * n), np.zeros(n, np.int64)
+    got = rt.lib.rt_ktime_read(rt.R, *(a.ctypes.data_as(P) for a in arrs), names, grid.ctypes.data_as(P), n)
+    rt.lib.rt_ktime(rt.R, 0)
+    return [names.raw[64 * i:64 * i + 64].split(b"\0")[0].decode() for i in range(got)]
+
+
+class Case:
+    """Two matrices and x on the device; run(kind, k, n) is one call on tokens [k, k + n)."""
+
+    def __init__(self, rt, rows, cols, t, seed, x=None, q8=None):
+        rng = np.random.default_rng(seed)
+        self.rt, self.rows, self.cols, self.t = rt, rows, cols, t
+        self.q8 = q8 or [synth.q8_rows(rng, rows, cols) for _ in range(2)]
+        self.x = synth.x_f32(rng, t, cols) if x is None else x
+        self.nw = (1.0 + 0.1 * rng.standard_normal(cols)).astype(np.float32)
+        self.res = rng.standard_normal((t, rows)).astype(np.float32)
+        self.w = [rt.upload(q, rows, cols) for q in self.q8]
+        self.p = {k: self.put(v) for k, v in (("x", self.x), ("nw", self.nw), ("res", self.res))}
+        self.y, self.z = rt.alloc(4 * t * rows), rt.alloc(4 * t * 16)
+
+    def put(self, a):
+        p = self.rt.alloc(a.nbytes)
+        self.rt.to_dev(p, a)
+        return p
+
+    def close(self):
+        for w in self.w:
+            self.rt.lib.rt_q8_free(self.rt.R, P(w))
+        for p in (*self.p.values(), self.y, self.z):
+            self.rt.free(p)
+
+    def run(self, kind, k, n):
+        lib, R, rows, cols, eps = self.rt.lib, self.rt.R, self.rows, self.cols, c.c_float(1e-6)
+        x, y, nw, res = P(self.p["x"] + 4 * k * cols), P(self.y + 4 * k * rows), P(self.p["nw"]), P(self.p["res"] + 4 * k * rows)
+        w = [P(v) for v in self.w]
+        if kind == "product":
+            lib.rt_gemm_dev(R, w[0], rows, cols, x, cols, n, y)
+        elif kind == "noalloc":
+            lib.rt_gemm_dev_noalloc(R, w[0], rows, cols, x, cols, n, y)
+        elif kind == "residual":
+            lib.rt_gemm_residual_dev(R, w[0], rows, cols, x, cols, n, res, y)
+        elif kind == "norm":
+            lib.rt_gemm_norm_dev(R, w[0], rows, cols, x, cols, n, nw, eps, y)
+        elif kind == "pair":
+            lib.rt_gemv_swiglu_dev(R, w[0], w[1], rows, cols, x, cols, n, y)
+        elif kind == "pair_norm":
+            lib.rt_gemv_swiglu_norm_dev(R, w[0], w[1], rows, cols, x, cols, n, nw, eps, y)
+        else:  # rounds: the matrix and a 16-row prefix of the other
+            ws, rr = (P * 2)(self.w[0], self.w[1]), (c.c_long * 2)(rows, 16)
+            ys = (P * 2)(self.y + 4 * k * rows, self.z + 4 * k * 16)
+            if kind == "round":
+                lib.rt_gemv_round_dev(R, 2, ws, rr, cols, x, cols, n, ys)
+            else:
+                lib.rt_gemv_round_norm_dev(R, 2, ws, rr, cols, x, cols, n, nw, eps, ys)
+
+    def out(self):
+        y, z = np.empty((self.t, self.rows), np.float32), np.empty((self.t, 16), np.float32)
+        self.rt.from_dev(y, self.y)
+        self.rt.from_dev(z, self.z)
+        return y, z
+
+    def nan(self):
+        self.rt.to_dev(self.y, np.full((self.t, self.rows), np.nan, np.float32))
+        self.rt.to_dev(self.z, np.full((self.t, 16), np.nan, np.float32))
+
+    def whole_and_parts(self, kind):
+        """(kernel name, outputs of one call, outputs of 64-token calls; a last call holds 5 tokens or more)"""
+        self.nan()
+        names = kernels(self.rt, lambda: self.run(kind, 0, self.t))
+        one = self.out()
+        self.nan()
+        for k in range(0, self.t, 64):
+            k = min(k, max(0, self.t - 5))
+            self.run(kind, k, min(64, self.t - k))
+        return names[0], one, self.out()
+
+
+KINDS = ("product", "noalloc", "residual", "norm", "pair", "pair_norm", "round", "round_norm")
+# (rows, cols, tokens, forced K splits): the tiles' edges. 512 x 4096 rows fill the device with the
+# small tiles and 12288 with the large ones
+SHAPES = [(256, 64, 300, 0), (512, 96, 2000, 0), (1888, 1056, 131, 0), (1888, 1056, 500, 3), (4096, 1024, 513, 1), (5136, 2784, 300, 0),
+          (12288, 1024, 512, 0), (12288, 1024, 257, 3), (12272, 1056, 250, 0), (16400, 512, 1030, 0)]
+
+
+@pytest.mark.parametrize("rows,cols,t,ks", SHAPES)
+def test_long_prompt_bits(rt, rows, cols, t, ks):
+    case = Case(rt, rows, cols, t, rows + cols + t)
+    rt.gemm_force(False, ks)
+    try:
+        for kind in KINDS:
+            name, one, parts = case.whole_and_parts(kind)
+            print("long prompt", rows, cols, t, ks, kind, name, flush=True)
+            for a, b in zip(one, parts):
+                assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), kind
+    finally:
+        rt.gemm_force()
+        case.close()
+
+
+def test_every_tile_runs_and_few_rows_do_not(rt):
+    """The configurations the rule chooses over sizes (each of the seven at least once), and matrices
+    of few rows on the 64-token launches, which split K over the device."""
+    seen = set()
+    for rows, cols, t in [(256, 64, 300), (4096, 1024, 512), (4096, 1024, 1024), (4096, 1024, 2048), (12288, 256, 512), (16384, 256, 1024), (2048, 512, 130)]:
+        case = Case(rt, rows, cols, t, 3)
+        try:
+            for kind in ("product", "pair"):
+                seen |= set(kernels(rt, lambda: case.run(kind, 0, t)))
+        finally:
+            case.close()
+    print(sorted(seen), flush=True)
+    assert {n for n in seen if n.startswith("gemm_tile<")} >= {f"gemm_tile<{v}>" for v in ("8, 2, 8, 1, 3", "4, 2, 8, 1, 4", "4, 1, 8, 1, 4", "4, 1, 4, 1, 3",
+                                                                                      "8, 1, 8, 2, 3", "4, 1, 8, 2, 4", "4, 1, 4, 2, 3")}
+    case = Case(rt, 16, 4096, 200, 4)
+    try:
+        assert kernels(rt, lambda: case.run("product", 0, 200))[0].startswith("gemm_mfma<")
+    finally:
+        case.close()
+
+
+def test_long_prompt_parity_and_image_chunks(rt, oracle):
+    """Against F64, with heavy-tailed scales; and a prompt whose limb image takes two chunks of
+    rt_gemm_dev_noalloc's 32 MiB (12288 columns: 384 tokens a chunk), bit for bit the one of 64 MiB."""
+    rng = np.random.default_rng(5)
+    q8 = synth.q8_rows(rng, 512, 12288, "lognormal")
+    case = Case(rt, 512, 12288, 450, 6, q8=[q8, q8])
+    try:
+        case.run("product", 0, 450)
+        whole = case.out()[0]
+        assert_parity(whole[:96], oracle.gemm_f64(q8, 512, 12288, case.x[:96]), "512x12288 t=450")
+        case.nan()
+        case.run("noalloc", 0, 450)
+        assert np.array_equal(case.out()[0].view(np.uint32), whole.view(np.uint32))
+    finally:
+        case.close()
+
+
+def test_long_prompt_non_finite(rt):
+    """Infinite and NaN x, and an infinite scale in a row's last block of an odd count: the same
+    values, NaN for NaN, as the 64-token launches."""
+    rows, cols, t = 256, 1056, 200
+    rng = np.random.default_rng(7)
+    q, d = synth.split(synth.q8_rows(rng, rows, cols), rows, cols)
+    d = d.copy()
+    d[3, -1], d[17, 5] = np.inf, np.inf
+    q8 = synth.join(q, d)
+    x = synth.x_f32(rng, t, cols)
+    x[0, 5], x[70, 40], x[150, cols - 1], x[199, 0] = np.inf, -np.inf, np.nan, 3e38
+    case = Case(rt, rows, cols, t, 8, x=x, q8=[q8, q8])
+    try:
+        for kind in ("product", "pair", "norm"):
+            name, one, parts = case.whole_and_parts(kind)
+            assert name.startswith("gemm_tile<"), name
+            assert np.array_equal(one[0], parts[0], equal_nan=True), kind
+    finally:
+        case.close()
+
+
+def test_long_prompt_recorded(q8rt, rt):
+    """Recorded and replayed three times with eager work between, bit for bit; and a runtime whose
+    limb image does not exist yet records the 64-token launches instead of refusing."""
+    case = Case(rt, 1024, 1024, 200, 9)
+    try:
+        case.run("pair", 0, 200)
+        case.run("product", 0, 200)
+        eager = case.out()[0]
+        rt.lib.rt_graph_begin(rt.R)
+        case.run("product", 0, 200)
+        g = rt.lib.rt_graph_end(rt.R)
+        for _ in range(3):
+            case.run("pair", 0, 200)
+            case.nan()
+            rt.lib.rt_graph_launch(rt.R, P(g))
+            assert np.array_equal(case.out()[0].view(np.uint32), eager.view(np.uint32))
+        rt.lib.rt_graph_free(rt.R, P(g))
+    finally:
+        case.close()
+    with q8rt.Runtime() as r2:
+        c2 = Case(r2, 1024, 1024, 200, 9)
+        c2.run("product", 0, 40)  # the 64-token launches' workspace, but no limb image
+        r2.lib.rt_graph_begin(r2.R)
+        c2.run("product", 0, 200)
+        g = r2.lib.rt_graph_end(r2.R)
+        c2.nan()
+        r2.lib.rt_graph_launch(r2.R, P(g))
+        assert np.array_equal(c2.out()[0].view(np.uint32), eager.view(np.uint32))
+        r2.lib.rt_graph_free(r2.R, P(g))
+        c2.close()
