@@ -137,7 +137,7 @@ void rt_q8_row(const void *w, long cols, long row, float *z);
  * another's y sees it; rt_dev_sync waits for all of them. These are what a caller that keeps
  * its activations in HBM uses, and what the throughput figures time. */
 void rt_gemv_dev(struct rt *R, const void *w, long rows, long cols, const float *x, float *y);
-/* Y = X W^T, t tokens (1..64), X rows x_stride floats apart (x_stride >= cols, % 4 == 0). */
+/* Y = X W^T, t tokens, X rows x_stride floats apart (x_stride >= cols, % 4 == 0). */
 void rt_gemm_dev(struct rt *R, const void *w, long rows, long cols, const float *x, long x_stride, long t, float *y);
 /* rt_gemm_dev that allocates nothing, for callers that cannot call hipMalloc (code under HIP graph
  * capture, tight serving loops, harnesses that forbid allocation). No counterpart in the reference.
@@ -150,7 +150,7 @@ void rt_gemm_dev_noalloc(struct rt *R, const void *w, long rows, long cols, cons
 /* A round of n (1..RT_BATCH) products sharing x, none reading another's y: y[i] = X w[i]^T,
  * w[i] [rows[i] cols]. At t <= 4 one launch where the decode kernel takes the shapes; from 5
  * tokens, 64 at a time, one matrix-core launch for the products and one launch of their partial
- * sums (each product on its own K split). Each y has
+ * sums (each product on its own K split), or one launch for all of a long prompt. Each y has
  * the bits of its own single product. The device form of rt_gemv_q x n + rt_gemv_go, which uses
  * the same launches for queued products that share x (the DeltaNet quartet QKV/GATE/BETA/ALPHA,
  * src/apl/qwen35.apl:93-96; the attention layer's Q/K/V, qwen35.apl:117-119). */
@@ -163,8 +163,9 @@ void rt_gemv_swiglu_dev(struct rt *R, const void *wg, const void *wu, long rows,
 /* ---- the epilogues on either side of a product (additions; the reference computes them on its
  * host around the products: RMS = {⍺×⍵×(RMS_EPS+(+/⍵×⍵)÷≢⍵)*¯0.5}, src/apl/qwen35.apl:49, before a
  * layer's mixer and FFN, and the residual Z←X+… after them, qwen35.apl:131-139). Fused into the
- * decode kernel (t <= 4) for K = 2048, 4096, 6144 and 12288 and the residual into the
- * matrix-core product's for t >= 5; other shapes run the norm or the add as a kernel of its own. The
+ * decode kernel (t <= 4; the norm up to 8192 columns and at 12288, the residual up to 16384), the residual
+ * into the matrix-core product's for t >= 5 and the norm into a long prompt's (more than 64 tokens);
+ * otherwise the norm or the add runs as a kernel of its own. The
  * norm is s = 1 / sqrt(eps + sum_k x[k]^2 / cols) per token in F32, xn[k] = nw[k] * (x[k] * s); its
  * sum runs in a fixed order for a given shape, so results repeat bit for bit, and a fused and a
  * separate norm differ only by that order (an ulp or so of s). The residual is one F32 add of the

@@ -221,6 +221,11 @@ struct q8_epi {
  * kernel takes the shape (nothing launched; the caller runs the epilogue apart). */
 int q8_launch_gemv_epi(q8_stream_t stream, const void *w0, const void *w1, long rows, long cols, const float *x, long x_stride, long t, float *y,
                        q8_epi e);
+/* The decode kernels for any cols up to 16384 (q8_gemv_any.hip), t = 1..4: false when they do not take
+ * the shape (nothing launched). */
+bool q8_launch_gemv_any(q8_stream_t stream, const void *w0, const void *w1, long rows, long cols, const float *x, long x_stride, long t, float *y, q8_epi e);
+struct q8_round;
+bool q8_launch_round_any(q8_stream_t stream, const q8_round &r, long cols, const float *x, long x_stride, long t, q8_epi e);
 /* The RMS norm apart: xn [t cols] (rows cols floats apart) from x [t cols] (x_stride apart). */
 void q8_launch_rmsnorm(q8_stream_t stream, const float *x, long x_stride, long t, long cols, const float *nw, float eps, float *xn);
 /* y[i] = a[i] + b[i], i < n (y may be a or b). */
@@ -228,6 +233,7 @@ void q8_launch_add(q8_stream_t stream, const float *a, const float *b, long n, f
 /* A round of products sharing x as one launch (t <= 4, cols % 1024 == 0, every rows % 8 == 0):
  * 0, or -1 (nothing launched: the caller runs them one by one). */
 #define Q8_ROUND_MAX 8
+#define Q8_ROUND_RW 8 /* rows a workgroup of a decode round */
 struct q8_round {
     int n;
     const void *w[Q8_ROUND_MAX];

@@ -1,6 +1,8 @@
 /* q8_kernels.hip: the Q8_0 product kernels for gfx950 and their launchers.
  *
- *   gemv_s      decode, t = 1..4 tokens: HBM-bound (1.88 flop/B). Each wave owns RW rows
+ *   gemv_k      decode, t = 1..4 tokens, for cols a multiple of 1024 (q8_gemv.h; any other cols up to
+ *               16384 in q8_gemv_any.hip): HBM-bound (1.88 flop/B).
+ *   gemv_s      the same past 16384 columns: each wave owns RW rows
  *               of one 16-row group and the whole of K; each lane takes 16-column units
  *               (one 16-byte load of one row) 64 units apart, so a wave reads 1 KiB of a row
  *               per load. Per unit: 16 exact int8->f32 converts, shared by the t tokens, a
@@ -22,6 +24,7 @@
 #include <stdlib.h>
 
 #include "q8_device.h"
+#include "q8_gemv.h"
 
 /* ---------------------------------------------------------------- decode GEMV */
 
@@ -135,209 +138,6 @@ __global__ __launch_bounds__(64 * GEMV_WAVES) void gemv_s(const uint8_t *__restr
     }
 }
 
-/* The decode kernel for cols % 1024 == 0: a workgroup of NW waves owns RW rows and all of K;
- * wave w takes the K-slice [w*1024*S, (w+1)*1024*S), S steps of 64 16-column units (lane l:
- * units l + 64 s). Every load of a lane is issued before any arithmetic, x first and then the
- * weights row by row (loads retire in order, so row r's arithmetic waits for rows 0..r only), so
- * the whole matrix is in flight in the first round trip: the layer matrices are latency-bound
- * otherwise. Per unit: 16 exact int8->f32 converts shared by the MT tokens, a 16-step fma chain
- * per token, then acc = fma(s, d, acc) with the unit's block scale. The lanes' partials are summed
- * by q8_wave_sum_dpp, the NW waves' in LDS in wave order: the same order every run. */
-/* EPI: 0 none; 1 the RMS norm of x first (e.nw, e.eps); 2 y = e.res + the product (q8_epi). y and
- * e.res may be the same array: each element is read and then written by the one thread that owns it. */
-template <int MT, int RW, int S, int NW, int PAIR, int EPI>
-__device__ __forceinline__ void gemv_body(const uint8_t *__restrict__ w0, const uint8_t *__restrict__ w1, long rows, long cols, const float *__restrict__ x,
-                                          long x_stride, float *y, long r0, q8_epi e)
-{
-    constexpr int P = PAIR + 1;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const long u0 = (long)wave * 64 * S + lane;
-
-    float4 xv[MT][S][4];
-#pragma unroll
-    for (int m = 0; m < MT; m++)
-#pragma unroll
-        for (int s = 0; s < S; s++)
-#pragma unroll
-            for (int c = 0; c < 4; c++)
-                xv[m][s][c] = *(const float4 *)(x + m * x_stride + 16 * (u0 + 64 * s) + 4 * c);
-    /* the residual of the output this thread stores (thread k < RW*MT stores row k / MT, token
-     * k % MT; the others load one of those too, so the load is unconditional), issued with x so
-     * that it is not a memory latency at the kernel's end */
-    float rv = 0.0f;
-    if constexpr (EPI == 2) {
-        static_assert(NW > 1, "the residual epilogue stores from threads < RW * MT");
-        const int k = (int)threadIdx.x % (RW * MT);
-        rv = e.res[(long)(k % MT) * rows + r0 + k / MT];
-    }
-    /* the norm's weights, the lane's columns, issued with x before the matrix */
-    float4 nv[S][4];
-    if constexpr (EPI == 1) {
-#pragma unroll
-        for (int s = 0; s < S; s++)
-#pragma unroll
-            for (int c = 0; c < 4; c++)
-                nv[s][c] = *(const float4 *)(e.nw + 16 * (u0 + 64 * s) + 4 * c);
-        /* keep them there: left to itself the scheduler issues them after the matrix, and the
-         * products of x and the norm weights, which every fma needs, then wait for all of it */
-        __builtin_amdgcn_sched_barrier(0);
-    }
-    uint4 q[RW][P][S];
-    uint16_t dh[RW][P][S];
-#pragma unroll
-    for (int r = 0; r < RW; r++)
-#pragma unroll
-        for (int p = 0; p < P; p++) {
-            const uint8_t *w = p ? w1 : w0;
-            const uint8_t *wq = w + q8s_row_q(r0 + r, cols);
-            const uint16_t *wd = (const uint16_t *)(w + q8s_row_d(r0 + r, cols));
-#pragma unroll
-            for (int s = 0; s < S; s++) {
-                q[r][p][s] = *(const uint4 *)(wq + 16 * (u0 + 64 * s));
-                dh[r][p][s] = wd[(u0 + 64 * s) >> 1];
-            }
-        }
-    /* every load issued before any arithmetic: left to itself the scheduler sinks the last rows'
-     * loads past the first rows' arithmetic, and past the wait for x, so they start a memory round
-     * trip late (4096x12288 at one token 10.85 against 11.0 us, at three 13.3 against 13.5). Not
-     * for 16 rows at two tokens, where the scheduler's own order measured faster (4096x12288: 11.4
-     * against 11.6 us) */
-    if constexpr (!(MT == 2 && RW == 16))
-        __builtin_amdgcn_sched_barrier(0);
-
-    /* the norm: x <- nw * x at once, and per token the sum of x^2 (the lane's, then the wave's,
-     * left in LDS for the final reduction, whose barrier covers it); s = 1 / sqrt(eps + sum / cols)
-     * multiplies the outputs at the end, W (nw * x) s = W (nw * (x s)): no barrier before the
-     * arithmetic starts, and x and nw are dead once multiplied */
-    float ss[MT];
-    if constexpr (EPI == 1) {
-#pragma unroll
-        for (int m = 0; m < MT; m++) {
-            float a = 0.0f;
-#pragma unroll
-            for (int s = 0; s < S; s++)
-#pragma unroll
-                for (int c = 0; c < 4; c++) {
-                    const float4 v = xv[m][s][c], g = nv[s][c];
-                    a = __builtin_fmaf(v.x, v.x, a);
-                    a = __builtin_fmaf(v.y, v.y, a);
-                    a = __builtin_fmaf(v.z, v.z, a);
-                    a = __builtin_fmaf(v.w, v.w, a);
-                    xv[m][s][c] = make_float4(g.x * v.x, g.y * v.y, g.z * v.z, g.w * v.w);
-                }
-            ss[m] = q8_wave_sum_dpp(a);
-        }
-    }
-    /* the wave's RW*P*MT sums over its lanes (q8_wave_sums, padded to a power of two), each
-     * written to LDS once; then the NW waves' in wave order. CH: in chunks of up to 8 rows, each
-     * chunk's sums run while later rows' loads still arrive. The two forms give the same bits; the
-     * compiler allocates their registers differently, and each was measured where it is used:
-     * chunks for the pair at 2 tokens (20.0 against 21.2 us on 12288x4096) and for 16 rows at 3
-     * tokens (119 registers, where one block of sums spills: 13.7 against 14.4 us at 8 rows on
-     * 4096x12288); one block everywhere else (the pair at 1 token 18.0 against 18.5 us, 16 rows at
-     * 2 and 4 tokens 11.7 / 14.5 against 12.5 / 15.6). */
-    constexpr bool CH = (PAIR && MT == 2) || (MT == 3 && RW == 16);
-    constexpr int RC = CH && RW > 8 ? 8 : RW, VC = RC * P * MT, VP = q8_pow2ceil(VC);
-    __shared__ float red[NW][RW * P * MT];
-    __shared__ float nsum[EPI == 1 ? NW : 1][MT];
-    if constexpr (EPI == 1) {
-        if (lane == 0)
-#pragma unroll
-            for (int m = 0; m < MT; m++)
-                nsum[wave][m] = ss[m];
-    }
-    /* row r's sum of token m of matrix p over the lane's columns */
-    auto row_sum = [&](int r, int p, int m) {
-        float acc = 0.0f;
-#pragma unroll
-        for (int s = 0; s < S; s++) {
-            const uint32_t qw[4] = {q[r][p][s].x, q[r][p][s].y, q[r][p][s].z, q[r][p][s].w};
-            const float xs[16] = {xv[m][s][0].x, xv[m][s][0].y, xv[m][s][0].z, xv[m][s][0].w, xv[m][s][1].x, xv[m][s][1].y,
-                                  xv[m][s][1].z, xv[m][s][1].w, xv[m][s][2].x, xv[m][s][2].y, xv[m][s][2].z, xv[m][s][2].w,
-                                  xv[m][s][3].x, xv[m][s][3].y, xv[m][s][3].z, xv[m][s][3].w};
-            float sum = 0.0f;
-#pragma unroll
-            for (int j = 0; j < 16; j++)
-                sum = __builtin_fmaf(q8_s8(qw[j >> 2], j & 3), xs[j], sum);
-            acc = __builtin_fmaf(sum, q8_half(dh[r][p][s]), acc);
-        }
-        return acc;
-    };
-    /* a block of VC sums (rows [ch*RC, +RC)) over the lanes, into LDS */
-    auto lane_sums = [&](float (&vals)[VP], int ch) {
-#pragma unroll
-        for (int i = VC; i < VP; i++)
-            vals[i] = 0.0f;
-        q8_wave_sums<VP>(vals, lane);
-        if (q8_wave_sums_owner<VP>(lane)) {
-#pragma unroll
-            for (int k = 0; k < (VP >> q8_wave_sums_steps<VP>()); k++) {
-                const int g = q8_wave_sums_index<VP>(lane, k);
-                if (g < VC)
-                    red[wave][ch * VC + g] = vals[k];
-            }
-        }
-    };
-    if constexpr (CH) {
-#pragma unroll
-        for (int ch = 0; ch < RW / RC; ch++) {
-            float vals[VP];
-#pragma unroll
-            for (int rr = 0; rr < RC; rr++)
-#pragma unroll
-                for (int p = 0; p < P; p++)
-#pragma unroll
-                    for (int m = 0; m < MT; m++)
-                        vals[(rr * P + p) * MT + m] = row_sum(ch * RC + rr, p, m);
-            lane_sums(vals, ch);
-        }
-    } else {
-        float acc[RW][P][MT];
-#pragma unroll
-        for (int r = 0; r < RW; r++)
-#pragma unroll
-            for (int p = 0; p < P; p++)
-#pragma unroll
-                for (int m = 0; m < MT; m++)
-                    acc[r][p][m] = row_sum(r, p, m);
-        float vals[VP];
-#pragma unroll
-        for (int r = 0; r < RW; r++)
-#pragma unroll
-            for (int p = 0; p < P; p++)
-#pragma unroll
-                for (int m = 0; m < MT; m++)
-                    vals[(r * P + p) * MT + m] = acc[r][p][m];
-        lane_sums(vals, 0);
-    }
-    __syncthreads();
-    if (threadIdx.x < RW * MT) {
-        const int r = threadIdx.x / MT, m = threadIdx.x % MT;
-        float v[P];
-#pragma unroll
-        for (int p = 0; p < P; p++) {
-            v[p] = red[0][(r * P + p) * MT + m];
-#pragma unroll
-            for (int k = 1; k < NW; k++)
-                v[p] += red[k][(r * P + p) * MT + m];
-        }
-        if constexpr (EPI == 1) {
-            /* the token's sum of x^2 over the waves, in wave order */
-            float tot = nsum[0][m];
-#pragma unroll
-            for (int k = 1; k < NW; k++)
-                tot += nsum[k][m];
-            const float sc = 1.0f / sqrtf(e.eps + tot / (float)cols);
-#pragma unroll
-            for (int p = 0; p < P; p++)
-                v[p] *= sc;
-        }
-        const long i = m * rows + r0 + r;
-        const float o = PAIR ? q8_swiglu(v[0], v[P - 1]) : v[0];
-        y[i] = EPI == 2 ? rv + o : o;
-    }
-}
-
 template <int MT, int RW, int S, int NW, int PAIR>
 __global__ __launch_bounds__(64 * NW) void gemv_k(const uint8_t *__restrict__ w0, const uint8_t *__restrict__ w1, long rows, long cols,
                                                   const float *__restrict__ x, long x_stride, float *__restrict__ y)
@@ -441,7 +241,9 @@ static void gemv_go(hipStream_t s, const void *w0, const void *w1, long rows, lo
         if (done)
             return;
     }
-    /* any other cols (a multiple of 32): the loop over K */
+    /* any other cols (a multiple of 32), and past 16384 the loop over K */
+    if (q8_launch_gemv_any((q8_stream_t)s, w0, w1, rows, cols, x, xs, MT, y, q8_epi{}))
+        return;
     const long waves = rows / 4;
     Q8_LAUNCH(q8_time_name("gemv_s", 3, MT, 4, PAIR), (gemv_s<MT, 4, PAIR>), dim3((unsigned)((waves + GEMV_WAVES - 1) / GEMV_WAVES)), dim3(64 * GEMV_WAVES), s,
               a, b, rows, cols, x, xs, y);
@@ -472,7 +274,7 @@ void q8_launch_gemv(q8_stream_t stream, const void *w0, const void *w1, long row
 }
 
 /* ---- the epilogue kernels: the layer shapes' K (S = 1 and NW = 2, 4, 6, 12: K = 2048, 4096,
- * 6144, 12288) at 2, 4 or 8 rows a workgroup; any other shape runs its epilogue apart */
+ * 6144, 12288) at 2, 4 or 8 rows a workgroup; other shapes in q8_gemv_any.hip */
 template <int MT, int RW, int PAIR, int EPI>
 static bool gemv_epi_rw(hipStream_t s, int nw, long kb, const uint8_t *a, const uint8_t *b, long rows, long cols, const float *x, long xs, float *y,
                         const q8_epi &e)
@@ -504,14 +306,15 @@ static bool gemv_epi_go(hipStream_t s, const void *w0, const void *w1, long rows
      * round of fewer, longer workgroups) is the faster shape then (12288x4096: 20.5 against 21.3 us) */
     if (PAIR && EPI == 1 && rw == 4 && rows % 8 == 0 && rows / 8 * nw >= 2048)
         rw = 8;
-    if (!kb || rows % rw)
-        return false;
-    switch (rw) {
-    case 2: return gemv_epi_rw<MT, 2, PAIR, EPI>(s, nw, kb, a, b, rows, cols, x, xs, y, e);
-    case 4: return gemv_epi_rw<MT, 4, PAIR, EPI>(s, nw, kb, a, b, rows, cols, x, xs, y, e);
-    case 8: return gemv_epi_rw<MT, 8, PAIR, EPI>(s, nw, kb, a, b, rows, cols, x, xs, y, e);
-    default: return false;
-    }
+    bool done = false;
+    if (kb && rows % rw == 0)
+        switch (rw) {
+        case 2: done = gemv_epi_rw<MT, 2, PAIR, EPI>(s, nw, kb, a, b, rows, cols, x, xs, y, e); break;
+        case 4: done = gemv_epi_rw<MT, 4, PAIR, EPI>(s, nw, kb, a, b, rows, cols, x, xs, y, e); break;
+        case 8: done = gemv_epi_rw<MT, 8, PAIR, EPI>(s, nw, kb, a, b, rows, cols, x, xs, y, e); break;
+        default: break;
+        }
+    return done || q8_launch_gemv_any((q8_stream_t)s, w0, w1, rows, cols, x, xs, MT, y, e);
 }
 
 template <int MT>
@@ -595,13 +398,12 @@ static bool round_go(hipStream_t s, int nw, long kb, const q8_round &r, long col
     return false;
 }
 
-constexpr int ROUND_RW = 8;
 
 /* the round's table and waves; false when the kernel does not take the shape */
 static bool round_plan(int n, const void *const *w, const long *rows, long cols, long t, float *const *y, q8_round &r, int &nw, long &kb)
 {
-    kb = cols % 1024 ? 0 : cols / 1024;
-    if (n < 1 || n > Q8_ROUND_MAX || t < 1 || t > 4 || !kb)
+    kb = cols % 1024 ? 0 : cols / 1024; /* 0: the instances for any cols */
+    if (n < 1 || n > Q8_ROUND_MAX || t < 1 || t > 4)
         return false;
     nw = (int)kb;
     if (kb > 16 || kb == 3 || kb == 5 || kb == 7 || (kb > 8 && kb != 12 && kb != 16))
@@ -609,12 +411,12 @@ static bool round_plan(int n, const void *const *w, const long *rows, long cols,
     r = q8_round{};
     r.n = n;
     for (int i = 0; i < n; i++) {
-        if (rows[i] % ROUND_RW)
+        if (rows[i] % Q8_ROUND_RW)
             return false;
         r.w[i] = w[i];
         r.y[i] = y[i];
         r.rows[i] = rows[i];
-        r.start[i + 1] = r.start[i] + rows[i] / ROUND_RW;
+        r.start[i + 1] = r.start[i] + rows[i] / Q8_ROUND_RW;
     }
     return true;
 }
@@ -645,13 +447,13 @@ int q8_launch_gemv_round_epi(q8_stream_t stream, int n, const void *const *w, co
     if (!e.nw || e.res || !round_plan(n, w, rows, cols, t, y, r, nw, kb))
         return -1;
     hipStream_t s = (hipStream_t)stream;
-    constexpr int RW = ROUND_RW;
+    constexpr int RW = Q8_ROUND_RW;
     bool done = false;
     switch (t) {
-    case 1: done = round_norm_go<1, RW>(s, nw, kb, r, cols, x, x_stride, e); break;
-    case 2: done = round_norm_go<2, RW>(s, nw, kb, r, cols, x, x_stride, e); break;
-    case 3: done = round_norm_go<3, RW>(s, nw, kb, r, cols, x, x_stride, e); break;
-    default: done = round_norm_go<4, RW>(s, nw, kb, r, cols, x, x_stride, e); break;
+    case 1: done = round_norm_go<1, RW>(s, nw, kb, r, cols, x, x_stride, e) || q8_launch_round_any(stream, r, cols, x, x_stride, 1, e); break;
+    case 2: done = round_norm_go<2, RW>(s, nw, kb, r, cols, x, x_stride, e) || q8_launch_round_any(stream, r, cols, x, x_stride, 2, e); break;
+    case 3: done = round_norm_go<3, RW>(s, nw, kb, r, cols, x, x_stride, e) || q8_launch_round_any(stream, r, cols, x, x_stride, 3, e); break;
+    default: done = round_norm_go<4, RW>(s, nw, kb, r, cols, x, x_stride, e) || q8_launch_round_any(stream, r, cols, x, x_stride, 4, e); break;
     }
     return done ? 0 : -1;
 }
@@ -663,14 +465,14 @@ int q8_launch_gemv_round(q8_stream_t stream, int n, const void *const *w, const 
     long kb;
     if (!round_plan(n, w, rows, cols, t, y, r, nw, kb))
         return -1;
-    constexpr int RW = ROUND_RW;
+    constexpr int RW = Q8_ROUND_RW;
     hipStream_t s = (hipStream_t)stream;
     bool done = false;
     switch (t) {
-    case 1: done = round_go<1, RW>(s, nw, kb, r, cols, x, x_stride); break;
-    case 2: done = round_go<2, RW>(s, nw, kb, r, cols, x, x_stride); break;
-    case 3: done = round_go<3, RW>(s, nw, kb, r, cols, x, x_stride); break;
-    default: done = round_go<4, RW>(s, nw, kb, r, cols, x, x_stride); break;
+    case 1: done = round_go<1, RW>(s, nw, kb, r, cols, x, x_stride) || q8_launch_round_any(stream, r, cols, x, x_stride, 1, q8_epi{}); break;
+    case 2: done = round_go<2, RW>(s, nw, kb, r, cols, x, x_stride) || q8_launch_round_any(stream, r, cols, x, x_stride, 2, q8_epi{}); break;
+    case 3: done = round_go<3, RW>(s, nw, kb, r, cols, x, x_stride) || q8_launch_round_any(stream, r, cols, x, x_stride, 3, q8_epi{}); break;
+    default: done = round_go<4, RW>(s, nw, kb, r, cols, x, x_stride) || q8_launch_round_any(stream, r, cols, x, x_stride, 4, q8_epi{}); break;
     }
     return done ? 0 : -1;
 }

@@ -1,0 +1,69 @@
+"""The decode kernels for any cols (csrc/q8_gemv_any.hip): K from one block to 16384 that is no multiple
+of 1024, at the edges of the wave classes (4, 8, 12, 16 waves), with the last wave from one unit to
+full, against F64; a token's bits whatever the token count, a round's products as their own launches',
+the epilogues, and an infinite scale in the block that dead lanes load."""
+import ctypes as c
+
+import numpy as np
+import pytest
+
+import synth
+from parity import assert_parity
+from test_gpu_tile import Case, kernels
+
+pytestmark = pytest.mark.gpu
+P = c.c_void_p
+
+SHAPES = [(16, 32), (64, 96), (2048, 1056), (5136, 2784), (4096, 4064), (1888, 4128), (2048, 8160), (528, 8224), (1024, 12320), (512, 16352), (512, 12256),
+          (2048, 5120), (256, 15360), (1024, 1088), (2048, 4352), (64, 16384 - 32), (32, 14336 + 896)]
+
+
+def rms(x, nw, eps=1e-6):
+    x = x.astype(np.float64)
+    return (nw * x / np.sqrt(eps + (x * x).mean(axis=1, keepdims=True))).astype(np.float64)
+
+
+@pytest.mark.parametrize("rows,cols", SHAPES)
+def test_any_cols(rt, oracle, rows, cols):
+    case = Case(rt, rows, cols, 4, rows + cols)
+    try:
+        got = {}
+        for kind in ("product", "residual", "norm", "pair", "pair_norm", "round", "round_norm"):
+            for t in (4, 3, 2, 1):
+                case.nan()
+                name = kernels(rt, lambda: case.run(kind, 0, t))[0]
+                y, z = case.out()
+                if t == 4:
+                    got[kind] = y
+                    print("any cols", rows, cols, kind, name, flush=True)
+                assert np.array_equal(y[:t].view(np.uint32), got[kind][:t].view(np.uint32)), (kind, t)
+                if kind.startswith("round"):
+                    case.rt.lib.rt_gemm_dev(rt.R, P(case.w[1]), 16, cols, P(case.p["x"]), cols, t, P(case.z))
+                    if kind == "round":
+                        assert np.array_equal(case.out()[1][:t].view(np.uint32), z[:t].view(np.uint32)), t
+        assert np.array_equal(got["round"].view(np.uint32), got["product"].view(np.uint32))
+        assert np.array_equal(got["residual"].view(np.uint32), (case.res + got["product"]).view(np.uint32))
+        xn = rms(case.x, case.nw)
+        g, u = (oracle.gemm_f64(q, rows, cols, case.x) for q in case.q8)
+        gn, un = (oracle.gemm_f64(q, rows, cols, xn.astype(np.float32)) for q in case.q8)
+        for kind, want in (("product", g), ("pair", oracle.swiglu_f64(g, u)), ("norm", gn), ("round_norm", gn), ("pair_norm", oracle.swiglu_f64(gn, un))):
+            assert_parity(got[kind], want, f"{kind} {rows}x{cols}")
+    finally:
+        case.close()
+
+
+def test_any_cols_infinite_scale(rt):
+    """Dead lanes load unit 0: an infinite scale there reaches its own row as the looping sum of the
+    same blocks gives it (infinite, or NaN), and no other row."""
+    rows, cols = 64, 1056
+    rng = np.random.default_rng(3)
+    q, d = synth.split(synth.q8_rows(rng, rows, cols), rows, cols)
+    d = d.copy()
+    d[5, 0] = np.inf
+    case = Case(rt, rows, cols, 4, 11, q8=[synth.join(q, d)] * 2)
+    try:
+        case.run("product", 0, 4)
+        y = case.out()[0]
+        assert np.all(np.isinf(y[:, 5])) and np.all(np.isfinite(np.delete(y, 5, axis=1)))
+    finally:
+        case.close()
