@@ -301,12 +301,19 @@ static bool gemv_epi_go(hipStream_t s, const void *w0, const void *w1, long rows
     const uint8_t *a = (const uint8_t *)w0, *b = (const uint8_t *)w1;
     const long kb = cols % 1024 ? 0 : cols / 1024;
     int rw, nw;
-    gemv_choose(PAIR, 1, rows, kb, &rw, &nw); /* the fused-epilogue instances: as measured at one token */
+    /* the norm's instances: as measured at one token; the residual's as the product's at MT */
+    gemv_choose(PAIR, EPI == 2 ? MT : 1, rows, kb, &rw, &nw);
     /* the pair with the norm: its norm weights take more registers, and 8 rows a workgroup (one
      * round of fewer, longer workgroups) is the faster shape then (12288x4096: 20.5 against 21.3 us) */
     if (PAIR && EPI == 1 && rw == 4 && rows % 8 == 0 && rows / 8 * nw >= 2048)
         rw = 8;
     bool done = false;
+    if constexpr (EPI == 2 && MT > 1)
+        if (rw == 16) { /* K = 12288: 4096 x 12288 with the residual at 4 tokens 18.0 us on 8 rows; 2 us less a layer here */
+            Q8_LAUNCH(q8_time_name("gemv_ke", 6, MT, 16, 1, 12, 0, 2), (gemv_ke<MT, 16, 1, 12, 0, 2>), dim3((unsigned)(rows / 16)), dim3(64 * 12), s, a, b,
+                      rows, cols, x, xs, y, e);
+            return true;
+        }
     if (kb && rows % rw == 0)
         switch (rw) {
         case 2: done = gemv_epi_rw<MT, 2, PAIR, EPI>(s, nw, kb, a, b, rows, cols, x, xs, y, e); break;
