@@ -164,6 +164,27 @@ __device__ __forceinline__ void q8_wave_sums(float (&v)[V], int lane)
     }
 }
 
+/* a + the squares of v's four values, and the norm's sums of W waves (4, or 16, of which the last 8 are zero up to 2048 columns): the pieces of the RMS
+ * norm's sum, which every kernel that computes the norm apart from a product adds in one order */
+__device__ __forceinline__ float q8_norm_add(float4 v, float a)
+{
+    a = __builtin_fmaf(v.x, v.x, a);
+    a = __builtin_fmaf(v.y, v.y, a);
+    a = __builtin_fmaf(v.z, v.z, a);
+    return __builtin_fmaf(v.w, v.w, a);
+}
+template <int W>
+__device__ __forceinline__ float q8_norm_fold(const float *p)
+{
+    const float a = (p[0] + p[1]) + (p[2] + p[3]);
+    if constexpr (W == 4)
+        return a;
+    else if constexpr (W == 8)
+        return a + ((p[4] + p[5]) + (p[6] + p[7]));
+    else
+        return (a + ((p[4] + p[5]) + (p[6] + p[7]))) + (((p[8] + p[9]) + (p[10] + p[11])) + ((p[12] + p[13]) + (p[14] + p[15])));
+}
+
 /* SiLU(g) * u (src/apl/qwen35.apl:38; docs/model.md:29: Sig = 1 / (1 + exp(min(700, -g)))):
  * in binary32 exp(min(700, -g)) overflows to inf for -g > 88.7 exactly as exp(-g) does, so
  * the clamp changes nothing and is left out. */

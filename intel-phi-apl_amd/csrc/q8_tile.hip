@@ -29,12 +29,17 @@
 
 #include "q8_bf16.h"
 
+template <int V>
+struct tile_c {
+    static constexpr int value = V;
+};
+
 /* ---------------------------------------------------------------- the limb image */
 
 /* The limbs of token tile blockIdx.y's blocks [16 blockIdx.x, +16), one block a wave; lane L holds
  * token L & 15 and the columns KCOL(L >> 4) .. +7 of the block. What lies past t or past the last
  * block is zero. nw != NULL: of the RMS norm, nw[k] * (x[k] * s), s from the sum of x^2 in rmsnorm_k's
- * order (256 threads of 4 columns each, summed by wave and over the waves), a wave a token: every
+ * order (a thread's columns, the wave, the waves), a wave a token: every
  * workgroup of the tile sums its 16 tokens again, from the L2, which costs less than a launch of
  * its own (4.9 us at 512 tokens of 4096 columns, and its x written and read again). */
 #define XIMG_BLOCKS 16
@@ -48,22 +53,35 @@ __global__ __launch_bounds__(64 * XIMG_BLOCKS) void ximage_k(const float *__rest
     if (nw) {
         const long tok = 16 * (long)blockIdx.y + wave;
         const float *xr = x + (tok < t ? tok : t - 1) * xs;
-        float a[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-        for (long k = 4 * (long)lane; k < cols; k += 1024)
+        /* the lane's part of each of rmsnorm_k's waves */
+        auto sum = [&](auto wc) {
+            constexpr int W = decltype(wc)::value;
+            float a[W];
 #pragma unroll
-            for (int q = 0; q < 4; q++)
-                if (k + 256 * q < cols) {
-                    const float4 v = *(const float4 *)(xr + k + 256 * q);
-                    a[q] = __builtin_fmaf(v.x, v.x, a[q]);
-                    a[q] = __builtin_fmaf(v.y, v.y, a[q]);
-                    a[q] = __builtin_fmaf(v.z, v.z, a[q]);
-                    a[q] = __builtin_fmaf(v.w, v.w, a[q]);
-                }
+            for (int q = 0; q < W; q++)
+                a[q] = 0.0f;
+            for (long k = 4 * (long)lane; k < cols; k += 256 * W) {
+                float4 v[W];
 #pragma unroll
-        for (int q = 0; q < 4; q++)
-            a[q] = q8_wave_sum_dpp(a[q]);
-        if (lane == 0)
-            scale[wave] = 1.0f / sqrtf(eps + ((a[0] + a[1]) + (a[2] + a[3])) / (float)cols);
+                for (int q = 0; q < W; q++)
+                    v[q] = *(const float4 *)(xr + (k + 256 * q < cols ? k + 256 * q : k));
+#pragma unroll
+                for (int q = 0; q < W; q++)
+                    if (k + 256 * q < cols)
+                        a[q] = q8_norm_add(v[q], a[q]);
+            }
+#pragma unroll
+            for (int q = 0; q < W; q++)
+                a[q] = q8_wave_sum_dpp(a[q]);
+            if (lane == 0)
+                scale[wave] = 1.0f / sqrtf(eps + q8_norm_fold<W>(a) / (float)cols);
+        };
+        if (cols <= 1024)
+            sum(tile_c<4>{});
+        else if (cols <= 2048)
+            sum(tile_c<8>{});
+        else
+            sum(tile_c<16>{});
         __syncthreads();
     }
     const int b = (int)blockIdx.x * XIMG_BLOCKS + wave;
@@ -104,10 +122,6 @@ struct tile_args {
     long cols, t;
 };
 
-template <int V>
-struct tile_c {
-    static constexpr int value = V;
-};
 typedef __attribute__((address_space(3))) void tile_lds;
 
 /* A workgroup of NW waves, MT token tiles x NW * RT row tiles (of each of the NP = 2 matrices of the
