@@ -315,7 +315,7 @@ void q8_gemm_split(long rows, long cols, q8_gemm_opts o, int *ks, int *cps);
  * and the launch: y[i] = X w[i]^T (plus res when given, n == 1), or pair_y = SiLU(G) * U. The bits
  * are those of the 64-token launches. */
 long q8_ximage_bytes(long t, long cols);
-bool q8_tile_takes(int n, const long *rows, long cols, long t, bool pair);
+bool q8_tile_takes(int n, const long *rows, long cols, long t, bool pair, q8_gemm_opts o);
 void q8_launch_ximage(q8_stream_t stream, const float *x, long x_stride, long t, long cols, const float *nw, float eps, void *img);
 void q8_launch_tile(q8_stream_t stream, int n, const void *const *w, const long *rows, long cols, long t, const void *img, float *const *y, const float *res,
                     float *pair_y, q8_gemm_opts o);

@@ -102,6 +102,9 @@ struct ctx {
     /* staging for the host-pointer products, in floats: pinned x and y, x's copy in HBM */
     float *hx = nullptr, *hy = nullptr, *dx = nullptr;
     size_t x_cap = 0, y_cap = 0;
+    /* y in HBM, for the calls whose products do not store it into hy themselves */
+    float *dy = nullptr;
+    size_t dy_cap = 0;
     /* the completion flag of the host-pointer calls (pinned) and the last number set in it */
     unsigned *flag = nullptr;
     unsigned flag_seq = 0;
@@ -338,7 +341,7 @@ bool on_matrix_cores(long t) { return t >= 5; }
  * Q8_GEMM_PART_MAX floats. Where not, the 64-token launches give the same bits. */
 bool tile_ready(ctx *c, int n, const long *rows, long cols, long t, bool pair, const float *part)
 {
-    if (!q8_tile_takes(n, rows, cols, t, pair) || q8_ximage_bytes(128, cols) > (part ? Q8_GEMM_PART_MAX * (long)sizeof(float) : TILE_IMG_BYTES))
+    if (!q8_tile_takes(n, rows, cols, t, pair, c->gemm_opts) || q8_ximage_bytes(128, cols) > (part ? Q8_GEMM_PART_MAX * (long)sizeof(float) : TILE_IMG_BYTES))
         return false;
     if (part || c->ximg)
         return true;
@@ -669,6 +672,19 @@ void run_round(ctx *c, job *jobs, int n, const char *what)
     bool direct = c->x_direct && !c->exact;
     for (int i = 0; i < n; i++)
         direct = direct && jobs[i].t <= 4;
+    /* Long prompts store y into HBM and a copy kernel moves it, a KiB a wave: the tiles' own stores are 64
+     * bytes of a token's row each, and over the host link they took 1077 us at 512 tokens of 12288 x
+     * 4096 against 868 for the 64-token launches' sums and 809 through the copy. */
+    bool far = false;
+    for (int i = 0; i < n; i++)
+        far = far || (jobs[i].t > 64 && !c->exact);
+    if (far && ny > c->dy_cap) {
+        if (c->dy)
+            HIPCHECK(hipFree(c->dy));
+        c->dy_cap = ny + ny / 2;
+        HIPCHECK(hipMalloc((void **)&c->dy, c->dy_cap * sizeof(float)));
+    }
+    float *yb = far ? c->dy : c->hy;
     const float *xb = c->dx;
     if (direct) {
         xb = c->hx;
@@ -687,7 +703,7 @@ void run_round(ctx *c, job *jobs, int n, const char *what)
         int idx[RT_BATCH], k = 0;
         for (int j = i; j < n; j++)
             if (!done[j] && jobs[j].x_off == jobs[i].x_off && jobs[j].t == jobs[i].t && jobs[j].cols == jobs[i].cols) {
-                w[k] = jobs[j].w, rows[k] = jobs[j].rows, y[k] = c->hy + jobs[j].y_off, idx[k++] = j;
+                w[k] = jobs[j].w, rows[k] = jobs[j].rows, y[k] = yb + jobs[j].y_off, idx[k++] = j;
             }
         if (k > 1 && round_launch(c, k, w, rows, jobs[i].cols, xb + jobs[i].x_off, jobs[i].cols, jobs[i].t, y))
             for (int j = 0; j < k; j++)
@@ -696,7 +712,11 @@ void run_round(ctx *c, job *jobs, int n, const char *what)
     for (int i = 0; i < n; i++) {
         const job &j = jobs[i];
         if (!done[i])
-            product(c, j.w, nullptr, j.rows, j.cols, xb + j.x_off, j.cols, j.t, c->hy + j.y_off);
+            product(c, j.w, nullptr, j.rows, j.cols, xb + j.x_off, j.cols, j.t, yb + j.y_off);
+    }
+    if (far) {
+        q8_launch_copy((q8_stream_t)c->stream, c->hy, c->dy, (long)(ny / 4)); /* ny is a multiple of 64 floats */
+        launched("the copy of y");
     }
     wait_done(c, what);
     const double t3 = c->htime_on ? now_us() : 0.0;
@@ -782,6 +802,8 @@ void rt_fini(struct rt *R)
         HIPCHECK(hipHostFree(c->hy));
     if (c->dx)
         HIPCHECK(hipFree(c->dx));
+    if (c->dy)
+        HIPCHECK(hipFree(c->dy));
     if (c->flag)
         HIPCHECK(hipHostFree(c->flag));
     if (c->scratch)

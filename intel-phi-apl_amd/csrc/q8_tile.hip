@@ -124,8 +124,21 @@ struct tile_args {
 
 typedef __attribute__((address_space(3))) void tile_lds;
 
+/* A barrier that no memory access moves across in the compiler, and that waits for none: the callers
+ * say what has to be there (__syncthreads would also wait for the loads in flight) */
+__device__ __forceinline__ void tile_barrier()
+{
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::: "memory");
+}
+
 /* A workgroup of NW waves, MT token tiles x NW * RT row tiles (of each of the NP = 2 matrices of the
- * pair), all of K in steps of one pair of blocks.
+ * pair), all of K in steps of one pair of blocks. KG == 2: two such sets of waves on the same tile, one
+ * taking the even K splits and one the odd, each with its own stages; the second hands each split's
+ * sums to the first through LDS, which adds them in split order.
  *
  * A step is 2 MT units, each one token tile against the wave's TR = NP * RT row tiles for one block:
  * 3 TR MFMAs, with the next unit's three limb reads, the previous unit's 4 TR scale FMAs and a share
@@ -142,25 +155,29 @@ typedef __attribute__((address_space(3))) void tile_lds;
  * reads every wave has used before that barrier. Loads past the last pair repeat the last pair.
  *
  * 8 waves, two a SIMD, each hiding the other's waits: 4 waves with twice the row tiles measured
- * slower (246 against 214 us), and so did 6 (unequal SIMDs: a pair at 512 tokens 299 us with 33 %
- * fewer idle workgroup slots against 305). */
-template <int MT, int RT, int NW, int NP, int NB>
-__global__ __launch_bounds__(64 * NW) void gemm_tile(tile_args a)
+ * slower (246 against 214 us), and 6 no faster (unequal SIMDs). */
+template <int MT, int RT, int NW, int NP, int NB, int KG>
+__global__ __launch_bounds__(64 * NW * KG) void gemm_tile(tile_args a)
 {
     constexpr int TR = NP * RT;
+    constexpr int WB = NB == 2 ? 3 : NB; /* weight sets: pair c's weights are issued in step c - WB + 1 */
     constexpr int SN = MT * 384;    /* 16-byte words of a stage */
     constexpr int SI = MT * 6 / NW; /* its 1 KiB loads a wave */
-    static_assert(MT * 6 % NW == 0 && NB >= 3 && NB <= 4, "a stage divides among the waves");
-    /* separate arrays, so that the reads of one do not wait for the loads of another */
-    __shared__ uint4 s0[SN], s1[SN], s2[SN], s3[NB > 3 ? SN : 1];
-    uint4 *bufs[NB];
-    bufs[0] = s0;
-    bufs[1] = s1;
-    bufs[2] = s2;
-    if constexpr (NB > 3)
-        bufs[3] = s3;
+    static_assert(MT * 6 % NW == 0 && NB >= 2 && NB <= 4 && (KG == 1 || KG == 2), "a stage divides among the waves");
+    /* separate arrays, so that the reads of one do not wait for the loads of another; each K group has
+     * its half */
+    __shared__ uint4 s0[KG * SN], s1[KG * SN], s2[NB > 2 ? KG * SN : 1], s3[NB > 3 ? KG * SN : 1];
+    __shared__ f32x4 ex[KG > 1 ? TR * MT * NW * 64 : 1]; /* group 1's split on its way to group 0 */
     const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int kg = KG > 1 ? wid / NW : 0, wave = KG > 1 ? wid % NW : wid;
+    uint4 *bufs[NB];
+    bufs[0] = s0 + kg * SN;
+    bufs[1] = s1 + kg * SN;
+    if constexpr (NB > 2)
+        bufs[2] = s2 + kg * SN;
+    if constexpr (NB > 3)
+        bufs[3] = s3 + kg * SN;
     const int nb = (int)(a.cols / Q8_BLOCK), np = (nb + 1) / 2;
     const int n = lane & 15, kq = lane >> 4;
     /* workgroups b, b + 8, ... share an XCD: the token groups of a row tile sit there next to each
@@ -210,22 +227,34 @@ __global__ __launch_bounds__(64 * NW) void gemm_tile(tile_args a)
         S.q[k] = *(const uint4 *)(wq[k] + (woff + 64u * (unsigned)c));
         S.d[k] = ((const u32u *)(wd[k] + (doff + (unsigned)(4 * c < 2 * nb - 4 ? 4 * c : 2 * nb - 4))))->v;
     };
-    /* block h of pair c as MFMA operands: lanes 0-31 hold block 2c, 32-63 block 2c + 1 (q8_bf16.h).
-     * The block past an odd count needs no mask: its limbs are zero and its weights finite, and its
-     * scale becomes 0 (the row's last scale is the high half of that load) */
+    /* block h of pair c as MFMA operands, in pieces of a few VALU instructions that spread over the
+     * units (all of a row tile's at once kept both waves of a SIMD on the VALU at the same time):
+     * piece 0 the row's scale, and for block 0 the pair's halves traded in place, lanes 0-31 hold block
+     * 2c and 32-63 block 2c + 1 (q8_bf16.h); pieces 1 to 4 two values a lane each. The block past
+     * an odd count needs no mask: its limbs are zero and its weights finite, and its scale becomes 0
+     * (the row's last scale is the high half of that load) */
     struct ops {
-        bf16x8 wb[TR];
+        uint32_t wb[TR][4];
         float d[TR];
     };
+    constexpr int CP = 5;
     const int odd = nb & 1;
-    auto conv1 = [&](ops &O, const wset &S, int k, int h, int c) __attribute__((always_inline)) {
-        const auto s02 = __builtin_amdgcn_permlane32_swap(S.q[k].x, S.q[k].z, false, false);
-        const auto s13 = __builtin_amdgcn_permlane32_swap(S.q[k].y, S.q[k].w, false, false);
-        O.wb[k] = q8_bf16(s02[h], s13[h]);
-        const uint32_t dd = S.d[k] >> (odd && c == np - 1 ? 16 : 0);
-        float d = q8_half((uint16_t)(h ? dd >> 16 : dd));
-        asm("" : "+v"(d)); /* converted once here, not in each of its FMAs */
-        O.d[k] = d;
+    auto conv1 = [&](ops &O, wset &S, int k, int h, int c, int piece) __attribute__((always_inline)) {
+        if (piece == 0) {
+            if (h == 0) {
+                const auto s02 = __builtin_amdgcn_permlane32_swap(S.q[k].x, S.q[k].z, false, false);
+                const auto s13 = __builtin_amdgcn_permlane32_swap(S.q[k].y, S.q[k].w, false, false);
+                S.q[k] = make_uint4(s02[0], s13[0], s02[1], s13[1]);
+            }
+            const uint32_t dd = S.d[k] >> (odd && c == np - 1 ? 16 : 0);
+            float d = q8_half((uint16_t)(h ? dd >> 16 : dd));
+            asm("" : "+v"(d)); /* converted once here, not in each of its FMAs */
+            O.d[k] = d;
+        } else {
+            const int i = piece - 1;
+            const uint32_t v = h ? (i < 2 ? S.q[k].z : S.q[k].w) : (i < 2 ? S.q[k].x : S.q[k].y);
+            O.wb[k][i] = pack_hi((float)(int8_t)(v >> (16 * (i & 1))), (float)(int8_t)(v >> (16 * (i & 1) + 8)));
+        }
     };
     auto lread = [&](uint4 (&xa)[3], const uint4 *buf, int m, int h) __attribute__((always_inline)) {
 #pragma unroll
@@ -239,32 +268,79 @@ __global__ __launch_bounds__(64 * NW) void gemm_tile(tile_args a)
 #pragma unroll
         for (int m = 0; m < MT; m++)
             acc[k][m] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    int left = spl; /* pairs to the end of the split */
-    bool first = true;
+    /* Steps: KG == 1, the pairs in order; KG == 2, group g's splits g, g + 2, ... in order, both groups in
+     * step, so a step is at pair c of the group, r pairs into its split. pos[k]: where step + k is */
+    struct place {
+        int c, r;
+    };
+    auto next = [&](place q) __attribute__((always_inline)) {
+        const bool end = q.r + 1 == spl;
+        return place{q.c + 1 + (KG > 1 && end ? spl : 0), end ? 0 : q.r + 1};
+    };
+    place pos[4];
+    pos[0] = place{kg * spl, 0};
+#pragma unroll
+    for (int k = 1; k < 4; k++)
+        pos[k] = next(pos[k - 1]);
+    const int splits = (np + spl - 1) / spl;
+    const int steps = KG == 1 ? np : splits % 2 ? splits / 2 * spl + np - (splits - 1) * spl : splits / 2 * spl;
+    auto clamp = [&](int c) __attribute__((always_inline)) { return c < np ? c : np - 1; };
+    bool first = true, pend = false; /* pend: group 1 has put a split into ex */
+    auto put_ex = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < TR; k++)
+#pragma unroll
+            for (int m = 0; m < MT; m++)
+                ex[((k * MT + m) * NW + wave) * 64 + lane] = acc[k][m];
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_waitcnt(0xc07f); /* lgkmcnt(0): in LDS before the next barrier */
+    };
+    auto add_ex = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < TR; k++)
+#pragma unroll
+            for (int m = 0; m < MT; m++) {
+                const f32x4 v = ex[((k * MT + m) * NW + wave) * 64 + lane];
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    tot[k][m][j] += v[j];
+            }
+    };
+    /* the end of a split: its sums join the splits' before it. Group 1's go through ex, which group 0
+     * reads in the next step (two steps at least before the next write: a split has two pairs or more) */
     auto fold = [&]() __attribute__((always_inline)) {
-        if (--left == 0) {
+        if (pos[0].r + 1 == spl) {
+            if (KG > 1 && kg) {
+                put_ex();
+            } else {
+#pragma unroll
+                for (int k = 0; k < TR; k++)
+#pragma unroll
+                    for (int m = 0; m < MT; m++)
+#pragma unroll
+                        for (int j = 0; j < 4; j++)
+                            tot[k][m][j] = first ? acc[k][m][j] : tot[k][m][j] + acc[k][m][j];
+                first = false;
+                pend = KG > 1 && pos[0].c + spl < np; /* group 1 ends a whole split in this step too */
+            }
 #pragma unroll
             for (int k = 0; k < TR; k++)
 #pragma unroll
-                for (int m = 0; m < MT; m++) {
-#pragma unroll
-                    for (int j = 0; j < 4; j++)
-                        tot[k][m][j] = first ? acc[k][m][j] : tot[k][m][j] + acc[k][m][j];
+                for (int m = 0; m < MT; m++)
                     acc[k][m] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-                }
-            first = false;
-            left = spl;
         }
     };
     ops O[2];
-    wset W[NB];
-    /* step c: limbs in bufs[I % NB], weights in W[I % NB], block 0's operands in O[I & 1]; during block
+    wset W[WB];
+    /* a step: limbs in bufs[I % NB], weights in W[I % WB], block 0's operands in O[I & 1]; during block
      * 0 block 1's are made, during block 1 the next pair's block 0's */
-    auto step = [&](auto Ic, int c) __attribute__((always_inline)) {
+    auto step = [&](auto Ic) __attribute__((always_inline)) {
         constexpr int I = decltype(Ic)::value, U = 2 * MT;
         constexpr int LP = (SI + TR + U - 3) / (U - 2); /* of the SI + TR groups of loads a unit */
-        constexpr int EV = MT / (TR + 1) < 1 ? 1 : MT / (TR + 1);
-        const int cn = c + NB - 1 < np ? c + NB - 1 : np - 1, c1 = c + 1 < np ? c + 1 : np - 1;
+        constexpr int PU = (CP * TR + MT - 1) / MT;                  /* conversion pieces a unit */
+        constexpr int VU = (4 * TR + 3 * PU + 3 * TR - 1) / (3 * TR); /* VALU instructions an MFMA */
+        const int c = pos[0].c, c1 = clamp(pos[1].c), cn = clamp(pos[NB - 1].c), cw = clamp(pos[WB - 1].c);
         ops O1;
         uint4 xa[2][3];
         f32x4 pv[2][TR];
@@ -279,7 +355,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_tile(tile_args a)
                 if (k < SI)
                     stage1(bufs[(I + NB - 1) % NB], cn, k);
                 else if (k < SI + TR)
-                    wload1(W[(I + NB - 1) % NB], cn, k - SI);
+                    wload1(W[(I + WB - 1) % WB], cw, k - SI);
             }
             const ops &OC = h ? O1 : O[I & 1];
             f32x4(&r)[TR] = pv[u & 1];
@@ -288,7 +364,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_tile(tile_args a)
             for (int l = 0; l < 3; l++)
 #pragma unroll
                 for (int k = 0; k < TR; k++)
-                    r[k] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, xa[u & 1][l]), OC.wb[k],
+                    r[k] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, xa[u & 1][l]), __builtin_bit_cast(bf16x8, OC.wb[k]),
                                                                    l ? r[k] : f32x4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
             if (u > 0) {
                 const ops &OP = (u - 1) / MT ? O1 : O[I & 1];
@@ -299,20 +375,19 @@ __global__ __launch_bounds__(64 * NW) void gemm_tile(tile_args a)
                         acc[k][(u - 1) % MT][j] = __builtin_fmaf(q[k][j], OP.d[k], acc[k][(u - 1) % MT][j]);
             }
 #pragma unroll
-            for (int k = 0; k < TR; k++)
-                if (m == (1 + k * EV < MT ? 1 + k * EV : MT - 1)) {
-                    if (h == 0)
-                        conv1(O1, W[I % NB], k, 1, c);
-                    else
-                        conv1(O[(I + 1) & 1], W[(I + 1) % NB], k, 0, c1);
-                }
-            /* the order within the unit: the limb reads, the loads, then two VALU between MFMAs */
+            for (int k = m * PU; k < (m + 1) * PU && k < CP * TR; k++) {
+                if (h == 0)
+                    conv1(O1, W[I % WB], k / CP, 1, c, k % CP);
+                else
+                    conv1(O[(I + 1) & 1], W[(I + 1) % WB], k / CP, 0, c1, k % CP);
+            }
+            /* the order within the unit: the limb reads, the loads, then the VALU work between MFMAs */
             __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
             __builtin_amdgcn_sched_group_barrier(0x020, 2, 0);
 #pragma unroll
             for (int i = 0; i < 3 * TR; i++) {
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, VU, 0);
             }
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -323,48 +398,75 @@ __global__ __launch_bounds__(64 * NW) void gemm_tile(tile_args a)
                 acc[k][MT - 1][j] = __builtin_fmaf(pv[1][k][j], O1.d[k], acc[k][MT - 1][j]);
         fold();
     };
-    /* pairs 0 .. NB - 2 in flight, each its stage and then its weights, as the steps issue them */
-    auto fetch = [&](uint4 *buf, wset &S, int c) __attribute__((always_inline)) {
-        c = c < np ? c : np - 1;
+    /* the stages of the first NB - 1 pairs and the weights of WB - 1 in flight, each pair's stage and then
+     * its weights, as the steps issue them (NB == 2: a pair's weights come a step before its stage) */
+    auto fetch = [&](int k) __attribute__((always_inline)) {
         __builtin_amdgcn_sched_barrier(0);
+        if (k < NB - 1)
 #pragma unroll
-        for (int k = 0; k < SI; k++)
-            stage1(buf, c, k);
+            for (int i = 0; i < SI; i++)
+                stage1(bufs[k], clamp(pos[k].c), i);
         __builtin_amdgcn_sched_barrier(0);
+        const int q = NB == 2 ? k + 1 : k;
 #pragma unroll
-        for (int k = 0; k < TR; k++)
-            wload1(S, c, k);
+        for (int i = 0; i < TR; i++)
+            wload1(W[q], clamp(pos[q].c), i);
         __builtin_amdgcn_sched_barrier(0);
     };
-    fetch(bufs[0], W[0], 0);
-    fetch(bufs[1], W[1], 1);
-    if constexpr (NB > 3)
-        fetch(bufs[2], W[2], 2);
+    if constexpr (NB == 2)
 #pragma unroll
-    for (int k = 0; k < TR; k++)
-        conv1(O[0], W[0], k, 0, 0);
+        for (int i = 0; i < TR; i++)
+            wload1(W[0], clamp(pos[0].c), i);
+#pragma unroll
+    for (int k = 0; k < NB - 1; k++)
+        fetch(k);
+#pragma unroll
+    for (int k = 0; k < CP * TR; k++)
+        conv1(O[0], W[0], k / CP, 0, clamp(pos[0].c), k % CP);
     constexpr int VN = (NB - 2) * (SI + 2 * TR) + 2 * TR;
     static_assert(VN < 64, "vmcnt");
+    int done = 0;
 #define STEP(I)                                                                                                        \
     {                                                                                                                  \
         __builtin_amdgcn_sched_barrier(0);                                                                             \
         __builtin_amdgcn_s_waitcnt(0x0f70 | (VN & 15) | (VN >> 4 << 14)); /* vmcnt(VN) */                              \
-        __builtin_amdgcn_s_barrier();                                                                                  \
-        __builtin_amdgcn_sched_barrier(0);                                                                             \
-        step(tile_c<I>{}, c + (I));                                                                                    \
-        if (c + (I) + 1 >= np)                                                                                         \
+        tile_barrier();                                                                                                \
+        if (KG > 1 && pend) {                                                                                          \
+            add_ex();                                                                                                  \
+            pend = false;                                                                                              \
+        }                                                                                                              \
+        if (KG == 1 || pos[0].c < np) /* group 1's last split may be shorter, or missing */                            \
+            step(tile_c<I>{});                                                                                         \
+        pos[0] = pos[1];                                                                                               \
+        pos[1] = pos[2];                                                                                               \
+        pos[2] = pos[3];                                                                                               \
+        pos[3] = next(pos[3]);                                                                                         \
+        if (++done >= steps)                                                                                           \
             break;                                                                                                     \
     }
-    if constexpr (NB == 3)
-        for (int c = 0;; c += 6) {
+    if constexpr (NB < 4)
+        for (;;) {
             STEP(0) STEP(1) STEP(2) STEP(3) STEP(4) STEP(5)
         }
     else
-        for (int c = 0;; c += 4) {
+        for (;;) {
             STEP(0) STEP(1) STEP(2) STEP(3)
         }
 #undef STEP
-    const bool tail = left != spl; /* the last split is shorter: its sums are still in acc */
+    if constexpr (KG > 1) {
+        /* the last of group 1's splits: in ex since the last step, or, shorter than the others, still in
+         * its acc */
+        const bool rest = splits % 2 == 0 && np % spl != 0;
+        tile_barrier();
+        if (rest && kg)
+            put_ex();
+        tile_barrier();
+        if (kg)
+            return;
+        if (pend || rest)
+            add_ex();
+    }
+    const bool tail = steps % spl != 0; /* the last split is shorter: its sums are still in acc */
     float *y = a.y[p];
     const long rows = 16L * rtn;
 #pragma unroll
@@ -392,29 +494,32 @@ __global__ __launch_bounds__(64 * NW) void gemm_tile(tile_args a)
 
 /* ---------------------------------------------------------------- launchers */
 
-/* The instantiated tiles, as X(MT, RT, NW, NP, NB, least, us0, us1). For a product (NP 1) 256 rows x
- * 128 tokens, 256 x 64, 128 x 64, 64 x 64; for the fused pair 128 rows of both x 128 tokens, 128 x 64,
+/* The instantiated tiles, as X(MT, RT, NW, NP, NB, KG, us0, us1). For a product (NP 1) 256 rows x 128
+ * tokens, 256 x 64, 128 x 64, 64 x 64; for the fused pair 128 rows of both x 128 tokens, 128 x 64,
  * 64 x 64. The large tile does the most work a limb read and a converted weight; the small ones fill
- * the device where there are few tiles. A step (one pair of blocks) of a round of workgroups takes us0
- * + us1 f us, f the share of the compute units that hold one (the clock falls as they fill), and a
- * product at least `least` us a step. Measured, 1-6 rounds, f from 1/8 to 1, K = 2048 to 12288:
- * 256 x 128 2.04 at f <= 1/2, 2.63 at 3/4, 3.1 at 1; 256 x 64 1.25, 1.39, 1.67; 128 x 64 0.77, 0.86,
- * 0.98; 64 x 64 (two workgroups a unit) 0.67-0.74 up to 256 workgroups, 1.14 at 512, 1.75 at 768;
- * the pair 2.02, 2.42, 2.68; 1.47-1.58 at 3/4, 1.62 at 1; 1.7 at 384, 2.85 at 768, 5.45 at 1536. */
+ * the device where there are few tiles, with two K groups, so that a compute unit still holds 8 (for
+ * 64 x 64 4) waves of two row tiles each: one row tile a wave reads 1 KiB of limbs an MFMA, all that
+ * LDS gives. 4096 x 12288 at 512 tokens 157 us against 170 for 128 x 64 with one row tile on 8 waves
+ * and no K groups; 2048 x 6144 at 203 tokens 55 us against 68 for 64 x 64.
+ * A step (one pair of blocks; of both groups' one each) of a round of workgroups takes us0 + us1 f
+ * us, f the share of the compute units that hold one (the clock falls as they fill); one workgroup a
+ * unit. Measured, 1-6 rounds, f from 1/8 to 1, K = 2048 to 12288: 256 x 128 2.04 at f <= 1/2,
+ * 2.3-2.6 at 3/4, 3.1 at 1; 256 x 64 1.25, 1.39, 1.67; 128 x 64 1.53-1.58, 1.56, 1.63-1.80; 64 x 64
+ * 1.16-1.22, -, 1.19-1.25; the pair 2.02, 2.42, 2.68; 1.47-1.58 at 3/4, 1.62 at 1; 1.70-1.75. */
 #define TILE_CFGS(X)                                                                                                   \
-    X(8, 2, 8, 1, 3, 0.0, 1.70, 1.30)                                                                                  \
-    X(4, 2, 8, 1, 4, 0.0, 1.10, 0.45)                                                                                  \
-    X(4, 1, 8, 1, 4, 0.0, 0.70, 0.25)                                                                                  \
-    X(4, 1, 4, 1, 3, 0.67, 0.57, 0.0)                                                                                  \
-    X(8, 1, 8, 2, 3, 0.0, 1.75, 0.90)                                                                                  \
-    X(4, 1, 8, 2, 4, 0.0, 1.30, 0.30)                                                                                  \
-    X(4, 1, 4, 2, 3, 1.00, 0.93, 0.0)
+    X(8, 2, 8, 1, 3, 1, 1.60, 1.20)                                                                                    \
+    X(4, 2, 8, 1, 4, 1, 1.10, 0.45)                                                                                    \
+    X(4, 2, 4, 1, 2, 2, 1.45, 0.27)                                                                                    \
+    X(4, 2, 2, 1, 2, 2, 1.10, 0.12)                                                                                    \
+    X(8, 1, 8, 2, 3, 1, 1.75, 0.90)                                                                                    \
+    X(4, 1, 8, 2, 4, 1, 1.30, 0.30)                                                                                    \
+    X(4, 1, 4, 2, 2, 2, 1.60, 0.15)
 
 struct tile_cfg {
-    int mt, rt, nw, np, nb;
-    float least, us0, us1;
+    int mt, rt, nw, np, nb, kg;
+    float us0, us1;
 };
-#define CFG(M, R, N, P, B, L, U0, U1) {M, R, N, P, B, L##f, U0##f, U1##f},
+#define CFG(M, R, N, P, B, G, U0, U1) {M, R, N, P, B, G, U0##f, U1##f},
 static const tile_cfg TILES[] = {TILE_CFGS(CFG)};
 #undef CFG
 
@@ -441,16 +546,25 @@ static int tile_cus()
 }
 
 /* The configuration for n products (pair: the fused two) of t tokens with the least modelled time */
-static const tile_cfg *tile_plan(int n, const long *rows, long cols, long t, bool pair, float *us)
+static const tile_cfg *tile_plan(int n, const long *rows, long cols, long t, bool pair, q8_gemm_opts o, float *us)
 {
     const tile_cfg *best = nullptr;
+    const long pairs = (cols / Q8_BLOCK + 1) / 2;
+    long half = 0; /* steps with two K groups: the most of any product */
+    for (int i = 0; i < n; i++) {
+        int ks, cps;
+        q8_gemm_split(rows[i], cols, o, &ks, &cps);
+        const long spl = (long)Q8_SPLIT_PAIRS * cps, splits = (pairs + spl - 1) / spl;
+        const long k = splits % 2 ? splits / 2 * spl + pairs - (splits - 1) * spl : splits / 2 * spl;
+        half = k > half ? k : half;
+    }
     for (const tile_cfg &k : TILES) {
         if (k.np != (pair ? 2 : 1))
             continue;
         const long groups = ((t + 15) / 16 + k.mt - 1) / k.mt, wgs = tile_rows(k, n, rows) * groups;
         const long rounds = (wgs + tile_cus() - 1) / tile_cus();
         const float step = (float)rounds * (k.us0 + k.us1 * (float)wgs / (float)(rounds * tile_cus()));
-        const float cost = (float)((cols / Q8_BLOCK + 1) / 2) * (step > k.least ? step : k.least);
+        const float cost = (float)(k.kg == 2 ? half : pairs) * step;
         if (!best || cost < *us) {
             best = &k;
             *us = cost;
@@ -461,18 +575,19 @@ static const tile_cfg *tile_plan(int n, const long *rows, long cols, long t, boo
 
 long q8_ximage_bytes(long t, long cols) { return (t + 15) / 16 * ((cols / Q8_BLOCK + 1) / 2) * 6144; }
 
-bool q8_tile_takes(int n, const long *rows, long cols, long t, bool pair)
+bool q8_tile_takes(int n, const long *rows, long cols, long t, bool pair, q8_gemm_opts o)
 {
     /* a row of one block has no two scales to load at once */
     if (t <= 64 || cols < 2 * Q8_BLOCK || n < 1 || n > Q8_ROUND_MAX || (pair && (n != 2 || rows[0] != rows[1])))
         return false;
     /* Against the 64-token launches: measured 35, 34, 20, 21 and 14 us a launch at 12288 x 4096, 4096 x
      * 12288, 4096 x 4096, 2048 x 6144 and 2048 x 2048 (13 us and 0.44 a million weights;
-     * less below 1024 rows, a few workgroups and their sums: 8 us); the image takes 3.5 us, and
+     * less below 1024 rows, a few workgroups and their sums: 8 us), a last one of fewer tokens 0.55, 0.7
+     * and 0.85 of that up to 16, 32 and 48; the image takes 3.5 us, and
      * 0.2 a MiB of it from there (10.5 us at 36 MiB). Few rows leave most of the device idle here,
      * where the 64-token launches split K over it: 4096 x 12288 at 128 tokens 66 against 117 us. */
     float us = 0.0f;
-    if (!tile_plan(n, rows, cols, t, pair, &us))
+    if (!tile_plan(n, rows, cols, t, pair, o, &us))
         return false;
     float weights = 0.0f, all = 0.0f;
     for (int i = 0; i < n; i++) {
@@ -480,7 +595,9 @@ bool q8_tile_takes(int n, const long *rows, long cols, long t, bool pair)
         all += (float)rows[i];
     }
     const float mib = (float)q8_ximage_bytes(t, cols) / 1048576.0f;
-    return us + 3.5f + 0.2f * mib < (float)((t + 63) / 64) * (8.0f + (all < 1024.0f ? all / 1024.0f : 1.0f) * 5.0f + 0.44e-6f * weights);
+    const long last = t % 64;
+    const float launches = (float)(t / 64) + (last == 0 ? 0.0f : last <= 16 ? 0.55f : last <= 32 ? 0.7f : last <= 48 ? 0.85f : 1.0f);
+    return us + 3.5f + 0.2f * mib < launches * (8.0f + (all < 1024.0f ? all / 1024.0f : 1.0f) * 5.0f + 0.44e-6f * weights);
 }
 
 void q8_launch_ximage(q8_stream_t stream, const float *x, long x_stride, long t, long cols, const float *nw, float eps, void *img)
@@ -495,7 +612,7 @@ void q8_launch_tile(q8_stream_t stream, int n, const void *const *w, const long 
 {
     hipStream_t s = (hipStream_t)stream;
     float us = 0.0f;
-    const tile_cfg *k = tile_plan(n, rows, cols, t, pair_y != nullptr, &us);
+    const tile_cfg *k = tile_plan(n, rows, cols, t, pair_y != nullptr, o, &us);
     tile_args a{};
     a.n = n;
     for (int i = 0; i < n; i++) {
@@ -516,9 +633,9 @@ void q8_launch_tile(q8_stream_t stream, int n, const void *const *w, const long 
     const long tiles = tile_rows(*k, n, rows);
     const unsigned grid = (unsigned)((tiles + 7) / 8 * 8 * a.groups);
     bool done = false;
-#define GO(M, R, N, P, B, L, U0, U1)                                                                                          \
-    if (!done && k->mt == M && k->rt == R && k->nw == N && k->np == P) {                                               \
-        Q8_LAUNCH(q8_time_name("gemm_tile", 5, M, R, N, P, B), (gemm_tile<M, R, N, P, B>), dim3(grid), dim3(64 * N), s, a); \
+#define GO(M, R, N, P, B, G, U0, U1)                                                                                \
+    if (!done && k->mt == M && k->rt == R && k->nw == N && k->np == P && k->kg == G) {                                 \
+        Q8_LAUNCH(q8_time_name("gemm_tile", 6, M, R, N, P, B, G), (gemm_tile<M, R, N, P, B, G>), dim3(grid), dim3(64 * N * G), s, a); \
         done = true;                                                                                                   \
     }
     TILE_CFGS(GO)

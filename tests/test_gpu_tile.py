@@ -102,7 +102,7 @@ class Case:
 KINDS = ("product", "noalloc", "residual", "norm", "pair", "pair_norm", "round", "round_norm")
 # (rows, cols, tokens, forced K splits): the tiles' edges. 512 x 4096 rows fill the device with the
 # small tiles and 12288 with the large ones
-SHAPES = [(256, 64, 300, 0), (512, 96, 2000, 0), (1888, 1056, 131, 0), (1888, 1056, 500, 3), (4096, 1024, 513, 1), (5136, 2784, 300, 0),
+SHAPES = [(256, 64, 300, 0), (512, 96, 2000, 0), (1888, 1056, 131, 0), (1888, 1056, 500, 3), (1888, 1056, 200, 1), (2048, 6144, 203, 0), (2048, 2048, 203, 5), (4096, 1024, 513, 1), (5136, 2784, 300, 0),
           (12288, 1024, 512, 0), (12288, 1024, 257, 3), (12272, 1056, 250, 0), (16400, 512, 1030, 0)]
 
 
@@ -133,8 +133,9 @@ def test_every_tile_runs_and_few_rows_do_not(rt):
         finally:
             case.close()
     print(sorted(seen), flush=True)
-    assert {n for n in seen if n.startswith("gemm_tile<")} >= {f"gemm_tile<{v}>" for v in ("8, 2, 8, 1, 3", "4, 2, 8, 1, 4", "4, 1, 8, 1, 4", "4, 1, 4, 1, 3",
-                                                                                      "8, 1, 8, 2, 3", "4, 1, 8, 2, 4", "4, 1, 4, 2, 3")}
+    assert {n for n in seen if n.startswith("gemm_tile<")} >= {f"gemm_tile<{v}>" for v in ("8, 2, 8, 1, 3, 1", "4, 2, 8, 1, 4, 1", "4, 2, 4, 1, 2, 2",
+                                                                                      "4, 2, 2, 1, 2, 2", "8, 1, 8, 2, 3, 1", "4, 1, 8, 2, 4, 1",
+                                                                                      "4, 1, 4, 2, 2, 2")}
     case = Case(rt, 16, 4096, 200, 4)
     try:
         assert kernels(rt, lambda: case.run("product", 0, 200))[0].startswith("gemm_mfma<")
@@ -210,3 +211,26 @@ def test_long_prompt_recorded(q8rt, rt):
         assert np.array_equal(c2.out()[0].view(np.uint32), eager.view(np.uint32))
         r2.lib.rt_graph_free(r2.R, P(g))
         c2.close()
+
+
+@pytest.mark.parametrize("t", [65, 130, 300])
+def test_long_prompt_host_calls(rt, t):
+    """rt_gemm, and two products queued with another of one token, on host arrays: y goes through HBM at
+    more than 64 tokens; bit for bit the device products, with x and y sizes that grow and shrink."""
+    case = Case(rt, 1040, 1056, t, 21 + t)
+    try:
+        case.run("product", 0, t)
+        want = case.out()[0]
+        y = [np.full((t, 1040), np.nan, np.float32) for _ in range(3)]
+        x1, y1 = np.ascontiguousarray(case.x[:1]), np.full((1, 1040), np.nan, np.float32)
+        rt.gemm(case.w[0], 1040, 1056, case.x, t, y[0])
+        rt.gemm_q(case.w[0], 1040, 1056, case.x, t, y[1])
+        rt.gemv_q(case.w[1], 1040, 1056, x1, y1)
+        rt.gemm_q(case.w[0], 1040, 1056, case.x, t, y[2])
+        rt.gemv_go()
+        for a in y:
+            assert np.array_equal(a.view(np.uint32), want.view(np.uint32))
+        rt.lib.rt_gemv_dev(rt.R, P(case.w[1]), 1040, 1056, P(case.p["x"]), P(case.y))
+        assert np.array_equal(case.out()[0][0].view(np.uint32), y1[0].view(np.uint32))
+    finally:
+        case.close()
