@@ -309,13 +309,14 @@ long q8_gemm_round_part_floats(int n, const long *rows, long cols, long t, q8_ge
  * last may hold fewer), a function of the shape alone (o.ks > 0 forces it). */
 #define Q8_SPLIT_PAIRS 2
 void q8_gemm_split(long rows, long cols, q8_gemm_opts o, int *ks, int *cps);
-/* More than 64 tokens as one launch (q8_tile.hip): whether it takes n products sharing x (pair: the
- * fused pair, n == 2 of one shape) and is the faster route, from their sizes alone. Then the limb
+/* More than 64 tokens (rounds on a norm more than 32) as one launch (q8_tile.hip): whether it takes n
+ * products sharing x (pair: the fused pair, n == 2 of one shape; norm: on the RMS norm of x, which the
+ * image then holds) and is the faster route, from their sizes alone. Then the limb
  * image of x (of its RMS norm when nw != NULL) at img, q8_ximage_bytes(t, cols) bytes, below 2^31, 16-byte aligned,
  * and the launch: y[i] = X w[i]^T (plus res when given, n == 1), or pair_y = SiLU(G) * U. The bits
  * are those of the 64-token launches. */
 long q8_ximage_bytes(long t, long cols);
-bool q8_tile_takes(int n, const long *rows, long cols, long t, bool pair, q8_gemm_opts o);
+bool q8_tile_takes(int n, const long *rows, long cols, long t, bool pair, bool norm, q8_gemm_opts o);
 void q8_launch_ximage(q8_stream_t stream, const float *x, long x_stride, long t, long cols, const float *nw, float eps, void *img);
 void q8_launch_tile(q8_stream_t stream, int n, const void *const *w, const long *rows, long cols, long t, const void *img, float *const *y, const float *res,
                     float *pair_y, q8_gemm_opts o);

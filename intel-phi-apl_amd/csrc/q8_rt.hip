@@ -155,8 +155,8 @@ constexpr size_t KT_MAX = 16384;
  * hundreds of tokens hides behind its arithmetic. Of one size, so that a graph may record any shape
  * once one long product has run. */
 constexpr long TILE_IMG_BYTES = 64L << 20;
-/* Rounds run as one launch from 81 tokens, single products and the fused pair from 65: the tests
- * hold the rounds of 65 to 70 tokens to the 64-token round kernels by name. */
+/* Rounds (but those on a norm) run as one launch from 81 tokens, single products and the fused pair
+ * from 65: the tests hold the rounds of 17 to 70 tokens to the 64-token round kernels by name. */
 constexpr long TILE_ROUND_MIN = 81;
 
 /* The runtimes alive, in the order rt_init set them up; rt_q8_row takes no struct rt
@@ -336,12 +336,13 @@ void reserve_pair(ctx *c, long rows, long cols, long t, float **g, float **rp)
  * decode kernels, which take at most 4 tokens a launch. */
 bool on_matrix_cores(long t) { return t >= 5; }
 
-/* Whether these products of more than 64 tokens run as one launch (q8_tile.hip), and their workspace
+/* Whether these products run as one launch (q8_tile.hip: more than 64 tokens, rounds on a norm more
+ * than 32), and their workspace
  * is there: the library's, allocated at its first use outside a recording, or part, a caller's of
  * Q8_GEMM_PART_MAX floats. Where not, the 64-token launches give the same bits. */
-bool tile_ready(ctx *c, int n, const long *rows, long cols, long t, bool pair, const float *part)
+bool tile_ready(ctx *c, int n, const long *rows, long cols, long t, bool pair, bool norm, const float *part)
 {
-    if (!q8_tile_takes(n, rows, cols, t, pair, c->gemm_opts) || q8_ximage_bytes(128, cols) > (part ? Q8_GEMM_PART_MAX * (long)sizeof(float) : TILE_IMG_BYTES))
+    if (!q8_tile_takes(n, rows, cols, t, pair, norm, c->gemm_opts) || q8_ximage_bytes(128, cols) > (part ? Q8_GEMM_PART_MAX * (long)sizeof(float) : TILE_IMG_BYTES))
         return false;
     if (part || c->ximg)
         return true;
@@ -385,7 +386,7 @@ void gemm_tokens(ctx *c, const void *w, long rows, long cols, const float *x, lo
                  float *part = nullptr)
 {
     const q8_stream_t s = (q8_stream_t)c->stream;
-    if (tile_ready(c, 1, &rows, cols, t, false, part)) {
+    if (tile_ready(c, 1, &rows, cols, t, false, false, part)) {
         if (!part)
             reserve_gemm(c, rows, cols, 64); /* as the 64-token launches: a later recording may count on it */
         tile_run(c, 1, &w, &rows, cols, x, xs, t, &y, res, nullptr, nullptr, 0.0f, part);
@@ -449,7 +450,7 @@ void product(ctx *c, const void *w0, const void *w1, long rows, long cols, const
         const void *w2[2] = {w0, w1};
         const long r2[2] = {rows, rows};
         bool pair_done = true;
-        if (tile_ready(c, 2, r2, cols, t, true, nullptr)) {
+        if (tile_ready(c, 2, r2, cols, t, true, false, nullptr)) {
             tile_run(c, 2, w2, r2, cols, x, xs, t, nullptr, nullptr, y, nullptr, 0.0f, nullptr);
             launched("the fused pair");
             return;
@@ -512,7 +513,7 @@ void product_epi(ctx *c, const void *w0, const void *w1, long rows, long cols, c
         float *xn = reserve_epi(c, (size_t)(t * cols));
         const void *w2[2] = {w0, w1};
         const long r2[2] = {rows, rows};
-        if (!c->exact && !apart && tile_ready(c, w1 ? 2 : 1, r2, cols, t, w1 != nullptr, nullptr)) {
+        if (!c->exact && !apart && tile_ready(c, w1 ? 2 : 1, r2, cols, t, w1 != nullptr, true, nullptr)) {
             /* the norm in the limb image: the same sum and the same xn as apart. The workspaces as
              * product() reserves them: a later recording of fewer tokens may count on them */
             if (w1) {
@@ -566,7 +567,7 @@ bool round_launch(ctx *c, int n, const void *const *w, const long *rows, long co
         /* 64 tokens at a time (a token's bits do not depend on t) */
         float *rp = reserve_round(c, n, rows, cols, t);
         rc = 0;
-        if (t >= TILE_ROUND_MIN && tile_ready(c, n, rows, cols, t, false, nullptr)) {
+        if (t >= TILE_ROUND_MIN && tile_ready(c, n, rows, cols, t, false, false, nullptr)) {
             tile_run(c, n, w, rows, cols, x, xs, t, y, nullptr, nullptr, nullptr, 0.0f, nullptr);
             launched("the round");
             return true;
@@ -1172,7 +1173,7 @@ void rt_gemv_round_norm_dev(struct rt *R, int n, const void *const *w, const lon
             kt_cancel(c);
     }
     float *xn = reserve_epi(c, (size_t)(t * cols));
-    if (!c->exact && n > 1 && !c->epi_apart && t >= TILE_ROUND_MIN && tile_ready(c, n, rows, cols, t, false, nullptr)) {
+    if (!c->exact && n > 1 && !c->epi_apart && tile_ready(c, n, rows, cols, t, false, true, nullptr)) {
         reserve_round(c, n, rows, cols, t);
         long total = 0;
         for (int i = 0; i < n; i++)

@@ -162,8 +162,8 @@ __global__ __launch_bounds__(64 * NW * KG) void gemm_tile(tile_args a)
     constexpr int TR = NP * RT;
     constexpr int WB = NB == 2 ? 3 : NB; /* weight sets: pair c's weights are issued in step c - WB + 1 */
     constexpr int SN = MT * 384;    /* 16-byte words of a stage */
-    constexpr int SI = MT * 6 / NW; /* its 1 KiB loads a wave */
-    static_assert(MT * 6 % NW == 0 && NB >= 2 && NB <= 4 && (KG == 1 || KG == 2), "a stage divides among the waves");
+    constexpr int SI = (MT * 6 + NW - 1) / NW; /* its 1 KiB loads a wave */
+    static_assert(NB >= 2 && NB <= 4 && (KG == 1 || KG == 2), "the buffers and groups the steps are written for");
     /* separate arrays, so that the reads of one do not wait for the loads of another; each K group has
      * its half */
     __shared__ uint4 s0[KG * SN], s1[KG * SN], s2[NB > 2 ? KG * SN : 1], s3[NB > 3 ? KG * SN : 1];
@@ -206,12 +206,14 @@ __global__ __launch_bounds__(64 * NW * KG) void gemm_tile(tile_args a)
     }
     const unsigned woff = (unsigned)(n * a.cols + 16 * kq), doff = (unsigned)(2 * n * nb);
     const __amdgpu_buffer_rsrc_t irs = __builtin_amdgcn_make_buffer_rsrc((void *)a.img, 0, a.img_bytes, 0x00027000);
-    const unsigned istep = (unsigned)ttn * 6144, ioff = (unsigned)tt0 * 6144 + (unsigned)(wave * SI) * 1024;
+    const unsigned istep = (unsigned)ttn * 6144, ioff = (unsigned)tt0 * 6144;
     /* load i of the wave's share of pair c's stage. Token tiles past the last one read the next pair's
      * tiles, or zeros past the image's end: tokens that are not stored, and no token's sums see another's */
     auto stage1 = [&](uint4 *buf, int c, int i) __attribute__((always_inline)) {
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(irs, (tile_lds *)(buf + (wave * SI + i) * 64), 16, lane * 16, (int)((unsigned)c * istep + ioff + i * 1024),
-                                                 0, 0);
+        int u = wave * SI + i; /* where the stage does not divide, the last loads repeat its last KiB */
+        if constexpr (MT * 6 % NW != 0)
+            u = u < MT * 6 ? u : MT * 6 - 1;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(irs, (tile_lds *)(buf + u * 64), 16, lane * 16, (int)((unsigned)c * istep + ioff + u * 1024), 0, 0);
     };
     /* a row tile's weights of pair c, 16 bytes a lane, and its row's two scales as one load (2-byte
      * aligned where the row has an odd count of blocks; its last pair reads the two blocks before
@@ -495,8 +497,8 @@ __global__ __launch_bounds__(64 * NW * KG) void gemm_tile(tile_args a)
 /* ---------------------------------------------------------------- launchers */
 
 /* The instantiated tiles, as X(MT, RT, NW, NP, NB, KG, us0, us1). For a product (NP 1) 256 rows x 128
- * tokens, 256 x 64, 128 x 64, 64 x 64; for the fused pair 128 rows of both x 128 tokens, 128 x 64,
- * 64 x 64. The large tile does the most work a limb read and a converted weight; the small ones fill
+ * tokens, 256 x 64, 128 x 64, 64 x 64, 64 x 48 and 64 x 32; for the fused pair 128 rows of both x 128
+ * tokens, 128 x 64, 64 x 64 and 64 x 32. The large tile does the most work a limb read and a converted weight; the small ones fill
  * the device where there are few tiles, with two K groups, so that a compute unit still holds 8 (for
  * 64 x 64 4) waves of two row tiles each: one row tile a wave reads 1 KiB of limbs an MFMA, all that
  * LDS gives. 4096 x 12288 at 512 tokens 157 us against 170 for 128 x 64 with one row tile on 8 waves
@@ -505,15 +507,21 @@ __global__ __launch_bounds__(64 * NW * KG) void gemm_tile(tile_args a)
  * us, f the share of the compute units that hold one (the clock falls as they fill); one workgroup a
  * unit. Measured, 1-6 rounds, f from 1/8 to 1, K = 2048 to 12288: 256 x 128 2.04 at f <= 1/2,
  * 2.3-2.6 at 3/4, 3.1 at 1; 256 x 64 1.25, 1.39, 1.67; 128 x 64 1.53-1.58, 1.56, 1.63-1.80; 64 x 64
- * 1.16-1.22, -, 1.19-1.25; the pair 2.02, 2.42, 2.68; 1.47-1.58 at 3/4, 1.62 at 1; 1.70-1.75. */
+ * 1.16-1.22, -, 1.19-1.25; 64 x 48 1.04-1.08; 64 x 32 0.85-0.9, 1.35-1.39 for 1.5 workgroups a unit
+ * (two fit); the pair 2.02, 2.42, 2.68; 1.47-1.58 at 3/4, 1.62 at 1; 1.70-1.75; 1.26-1.48. 4096 x 4096 at
+ * 144 tokens 34.7 us on 64 x 48 tiles against 40.2 on 64 x 64, 6144 x 2048 at 64 16.6 on 64 x 32 against
+ * 21.9. */
 #define TILE_CFGS(X)                                                                                                   \
     X(8, 2, 8, 1, 3, 1, 1.60, 1.20)                                                                                    \
     X(4, 2, 8, 1, 4, 1, 1.10, 0.45)                                                                                    \
     X(4, 2, 4, 1, 2, 2, 1.45, 0.27)                                                                                    \
     X(4, 2, 2, 1, 2, 2, 1.10, 0.12)                                                                                    \
+    X(3, 2, 2, 1, 2, 2, 0.95, 0.08)                                                                                    \
+    X(2, 2, 2, 1, 2, 2, 0.72, 0.14)                                                                                    \
     X(8, 1, 8, 2, 3, 1, 1.75, 0.90)                                                                                    \
     X(4, 1, 8, 2, 4, 1, 1.30, 0.30)                                                                                    \
-    X(4, 1, 4, 2, 2, 2, 1.60, 0.15)
+    X(4, 1, 4, 2, 2, 2, 1.60, 0.15)                                                                                    \
+    X(2, 1, 4, 2, 2, 2, 1.15, 0.30)
 
 struct tile_cfg {
     int mt, rt, nw, np, nb, kg;
@@ -575,17 +583,18 @@ static const tile_cfg *tile_plan(int n, const long *rows, long cols, long t, boo
 
 long q8_ximage_bytes(long t, long cols) { return (t + 15) / 16 * ((cols / Q8_BLOCK + 1) / 2) * 6144; }
 
-bool q8_tile_takes(int n, const long *rows, long cols, long t, bool pair, q8_gemm_opts o)
+bool q8_tile_takes(int n, const long *rows, long cols, long t, bool pair, bool norm, q8_gemm_opts o)
 {
-    /* a row of one block has no two scales to load at once */
-    if (t <= 64 || cols < 2 * Q8_BLOCK || n < 1 || n > Q8_ROUND_MAX || (pair && (n != 2 || rows[0] != rows[1])))
+    /* up to 64 tokens only rounds on a norm, from three token tiles: the image takes the norm's launch in, and
+     * a round's many small splits leave the most partials to sum (the 9B DeltaNet quartet at 64
+     * tokens: norm, product and sums 59 us, image and tiles 42). Single products and the pair gain
+     * nothing (12288 x 4096 at 64 tokens 42 + 3.5 against 35, the pair 61 + 3.5 against 63) */
+    const bool few = t <= 64;
+    if ((few && (t <= 32 || n < 2 || pair || !norm)) || n < 1 || n > Q8_ROUND_MAX || (pair && (n != 2 || rows[0] != rows[1])))
         return false;
-    /* Against the 64-token launches: measured 35, 34, 20, 21 and 14 us a launch at 12288 x 4096, 4096 x
-     * 12288, 4096 x 4096, 2048 x 6144 and 2048 x 2048 (13 us and 0.44 a million weights;
-     * less below 1024 rows, a few workgroups and their sums: 8 us), a last one of fewer tokens 0.55, 0.7
-     * and 0.85 of that up to 16, 32 and 48; the image takes 3.5 us, and
-     * 0.2 a MiB of it from there (10.5 us at 36 MiB). Few rows leave most of the device idle here,
-     * where the 64-token launches split K over it: 4096 x 12288 at 128 tokens 66 against 117 us. */
+    /* a row of one block has no two scales to load at once */
+    if (cols < 2 * Q8_BLOCK)
+        return false;
     float us = 0.0f;
     if (!tile_plan(n, rows, cols, t, pair, o, &us))
         return false;
@@ -594,10 +603,19 @@ bool q8_tile_takes(int n, const long *rows, long cols, long t, bool pair, q8_gem
         weights += (float)rows[i] * (float)cols;
         all += (float)rows[i];
     }
-    const float mib = (float)q8_ximage_bytes(t, cols) / 1048576.0f;
+    /* Against the 64-token launches: measured 35, 34, 20, 21 and 14 us a launch at 12288 x 4096, 4096 x
+     * 12288, 4096 x 4096, 2048 x 6144 and 2048 x 2048 (13 us and 0.44 a million weights; less below
+     * 1024 rows, a few workgroups and their sums: 8 us), a last one of fewer tokens 0.55, 0.7 and 0.85
+     * of that up to 16, 32 and 48; a round 55, 43 and 29 at 50, 42 and 25 million weights (taken as 16 us
+     * and 0.5), its norm 3.5. The image takes 3.5 us, and 0.2 a MiB of it from there (10.5 us at 36
+     * MiB). Few rows leave most of the device idle here, where the 64-token launches split K over it:
+     * 4096 x 12288 at 128 tokens 66 against 117 us. */
+    us += 3.5f + 0.2f * (float)q8_ximage_bytes(t, cols) / 1048576.0f;
+    if (few)
+        return us < (t <= 48 ? 0.85f : 1.0f) * (16.0f + 0.5e-6f * weights) + 3.5f;
     const long last = t % 64;
     const float launches = (float)(t / 64) + (last == 0 ? 0.0f : last <= 16 ? 0.55f : last <= 32 ? 0.7f : last <= 48 ? 0.85f : 1.0f);
-    return us + 3.5f + 0.2f * mib < launches * (8.0f + (all < 1024.0f ? all / 1024.0f : 1.0f) * 5.0f + 0.44e-6f * weights);
+    return us < launches * (8.0f + (all < 1024.0f ? all / 1024.0f : 1.0f) * 5.0f + 0.44e-6f * weights);
 }
 
 void q8_launch_ximage(q8_stream_t stream, const float *x, long x_stride, long t, long cols, const float *nw, float eps, void *img)

@@ -122,10 +122,11 @@ def test_long_prompt_bits(rt, rows, cols, t, ks):
 
 
 def test_every_tile_runs_and_few_rows_do_not(rt):
-    """The configurations the rule chooses over sizes (each of the seven at least once), and matrices
+    """The configurations the rule chooses over sizes (each at least once), and matrices
     of few rows on the 64-token launches, which split K over the device."""
     seen = set()
-    for rows, cols, t in [(256, 64, 300), (4096, 1024, 512), (4096, 1024, 1024), (4096, 1024, 2048), (12288, 256, 512), (16384, 256, 1024), (2048, 512, 130)]:
+    for rows, cols, t in [(256, 64, 300), (4096, 1024, 512), (4096, 1024, 1024), (4096, 1024, 2048), (12288, 256, 512), (16384, 256, 1024), (2048, 512, 130), (4096, 1024, 144), (2048, 1024, 200),
+                          (1024, 512, 66), (4096, 512, 200)]:
         case = Case(rt, rows, cols, t, 3)
         try:
             for kind in ("product", "pair"):
@@ -135,8 +136,9 @@ def test_every_tile_runs_and_few_rows_do_not(rt):
     print(sorted(seen), flush=True)
     assert {n for n in seen if n.startswith("gemm_tile<")} >= {f"gemm_tile<{v}>" for v in ("8, 2, 8, 1, 3, 1", "4, 2, 8, 1, 4, 1", "4, 2, 4, 1, 2, 2",
                                                                                       "4, 2, 2, 1, 2, 2", "8, 1, 8, 2, 3, 1", "4, 1, 8, 2, 4, 1",
-                                                                                      "4, 1, 4, 2, 2, 2")}
-    case = Case(rt, 16, 4096, 200, 4)
+                                                                                      "4, 1, 4, 2, 2, 2", "3, 2, 2, 1, 2, 2", "2, 2, 2, 1, 2, 2",
+                                                                                      "2, 1, 4, 2, 2, 2")}
+    case = Case(rt, 16, 8192, 200, 4)
     try:
         assert kernels(rt, lambda: case.run("product", 0, 200))[0].startswith("gemm_mfma<")
     finally:
@@ -233,4 +235,26 @@ def test_long_prompt_host_calls(rt, t):
         rt.lib.rt_gemv_dev(rt.R, P(case.w[1]), 1040, 1056, P(case.p["x"]), P(case.y))
         assert np.array_equal(case.out()[0][0].view(np.uint32), y1[0].view(np.uint32))
     finally:
+        case.close()
+
+
+@pytest.mark.parametrize("rows,cols,t", [(12288, 4096, 64), (12288, 4096, 40), (6144, 1056, 33), (4096, 2048, 50)])
+def test_round_on_a_norm_up_to_64_tokens(rt, rows, cols, t):
+    """Rounds on a norm from 33 tokens: the norm in the limb image and the tiles, against the norm, the
+    64-token round and its sums apart, bit for bit (whichever the rule takes at these sizes)."""
+    case = Case(rt, rows, cols, t, rows + t)
+    try:
+        case.nan()
+        name = kernels(rt, lambda: case.run("round_norm", 0, t))[0]
+        got = case.out()
+        rt.set_epi_apart(True)
+        case.nan()
+        case.run("round_norm", 0, t)
+        rt.set_epi_apart(False)
+        print("round on a norm", rows, cols, t, name, flush=True)
+        assert rows != 12288 or t != 64 or name.startswith("gemm_tile<"), name
+        for a, b in zip(got, case.out()):
+            assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+    finally:
+        rt.set_epi_apart(False)
         case.close()
