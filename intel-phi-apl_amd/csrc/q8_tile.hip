@@ -50,9 +50,20 @@ __global__ __launch_bounds__(64 * XIMG_BLOCKS) void ximage_k(const float *__rest
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int nb = (int)(cols / Q8_BLOCK), np = (nb + 1) / 2;
     __shared__ float scale[16];
+    /* this wave's block, loaded before the norm's sum so that the two memory round trips overlap
+     * (traced at 64 tokens of 4096 columns on a norm 8.2 against 9.4 us) */
+    const int b = (int)blockIdx.x * XIMG_BLOCKS + wave;
+    const long tok = 16 * (long)blockIdx.y + (lane & 15);
+    const bool in = tok < t && b < nb;
+    const long k0 = (long)(b < nb ? b : nb - 1) * Q8_BLOCK + kcol(lane >> 4);
+    const float *px = x + (tok < t ? tok : t - 1) * xs + k0;
+    float4 a = *(const float4 *)px, c = *(const float4 *)(px + 4), g{}, e{};
     if (nw) {
-        const long tok = 16 * (long)blockIdx.y + wave;
-        const float *xr = x + (tok < t ? tok : t - 1) * xs;
+        g = *(const float4 *)(nw + k0);
+        e = *(const float4 *)(nw + k0 + 4);
+        __builtin_amdgcn_sched_barrier(0);
+        const long row = 16 * (long)blockIdx.y + wave;
+        const float *xr = x + (row < t ? row : t - 1) * xs;
         /* the lane's part of each of rmsnorm_k's waves */
         auto sum = [&](auto wc) {
             constexpr int W = decltype(wc)::value;
@@ -84,17 +95,10 @@ __global__ __launch_bounds__(64 * XIMG_BLOCKS) void ximage_k(const float *__rest
             sum(tile_c<16>{});
         __syncthreads();
     }
-    const int b = (int)blockIdx.x * XIMG_BLOCKS + wave;
     if (b >= 2 * np)
         return;
-    const long tok = 16 * (long)blockIdx.y + (lane & 15);
-    const bool in = tok < t && b < nb;
-    const long k0 = (long)(b < nb ? b : nb - 1) * Q8_BLOCK + kcol(lane >> 4);
-    const float *px = x + (tok < t ? tok : t - 1) * xs + k0;
-    float4 a = *(const float4 *)px, c = *(const float4 *)(px + 4);
     if (nw) {
         const float s = scale[lane & 15];
-        const float4 g = *(const float4 *)(nw + k0), e = *(const float4 *)(nw + k0 + 4);
         a = make_float4(g.x * (a.x * s), g.y * (a.y * s), g.z * (a.z * s), g.w * (a.w * s));
         c = make_float4(e.x * (c.x * s), e.y * (c.y * s), e.z * (c.z * s), e.w * (c.w * s));
     }
