@@ -38,8 +38,9 @@ __host__ __device__ inline int q8_any_waves(long cols)
 /* EPI: 0 none; 1 the RMS norm of x first (e.nw, e.eps); 2 y = e.res + the product (q8_epi). y and
  * e.res may be the same array: each element is read and then written by the one thread that owns it. */
 /* ANY: cols any multiple of 32, S = 1, the waves the launch gave (at most NW; q8_any_waves). With a
- * wave a started 1024 columns, a lane past the row's last unit loads unit 0 and counts as zero, x and
- * scale (its 0 * scale would be NaN for an infinite scale). With a wave a whole 1024 columns, the
+ * wave a started 1024 columns, a lane past the row's last unit loads unit 0 and counts as zero, x (after
+ * its product with the norm's weight: 0 times an infinite weight would be NaN) and scale (0 times an
+ * infinite scale would be, too). With a wave a whole 1024 columns, the
  * tail's units go to the workgroup's threads once more, a row and a unit each (every row and matrix
  * has TP neighbouring lanes, TP the power of two from its units up), and are added after the waves'
  * sums: 129 blocks would otherwise take a fifth wave for two units. */
@@ -120,14 +121,13 @@ __device__ __forceinline__ void gemv_body(const uint8_t *__restrict__ w0, const 
             td = ((const uint16_t *)(w + q8s_row_d(r0 + tr, cols)))[tu >> 1];
         }
     }
-    if constexpr (ANY) {
+    auto live4 = [&](float4 v) { return make_float4(live ? v.x : 0.0f, live ? v.y : 0.0f, live ? v.z : 0.0f, live ? v.w : 0.0f); };
+    if constexpr (ANY && EPI != 1) {
 #pragma unroll
         for (int m = 0; m < MT; m++)
 #pragma unroll
-            for (int c = 0; c < 4; c++) {
-                float4 &v = xv[m][0][c];
-                v = make_float4(live ? v.x : 0.0f, live ? v.y : 0.0f, live ? v.z : 0.0f, live ? v.w : 0.0f);
-            }
+            for (int c = 0; c < 4; c++)
+                xv[m][0][c] = live4(xv[m][0][c]);
     }
 
     /* the norm: x <- nw * x at once, and per token the sum of x^2 (the lane's, then the wave's,
@@ -148,9 +148,9 @@ __device__ __forceinline__ void gemv_body(const uint8_t *__restrict__ w0, const 
                     a = __builtin_fmaf(v.y, v.y, a);
                     a = __builtin_fmaf(v.z, v.z, a);
                     a = __builtin_fmaf(v.w, v.w, a);
-                    xv[m][s][c] = make_float4(g.x * v.x, g.y * v.y, g.z * v.z, g.w * v.w);
+                    xv[m][s][c] = live4(make_float4(g.x * v.x, g.y * v.y, g.z * v.z, g.w * v.w));
                 }
-            ss[m] = q8_wave_sum_dpp(a);
+            ss[m] = q8_wave_sum_dpp(live ? a : 0.0f);
         }
     }
     /* the wave's RW*P*MT sums over its lanes (q8_wave_sums, padded to a power of two), each
@@ -247,7 +247,6 @@ __device__ __forceinline__ void gemv_body(const uint8_t *__restrict__ w0, const 
 #pragma unroll
                 for (int c = 0; c < 4; c++) {
                     float4 v = *(const float4 *)(x + m * x_stride + 16 * tu + 4 * c);
-                    v = make_float4(tlive ? v.x : 0.0f, tlive ? v.y : 0.0f, tlive ? v.z : 0.0f, tlive ? v.w : 0.0f);
                     if constexpr (EPI == 1) {
                         const float4 g = *(const float4 *)(e.nw + 16 * tu + 4 * c);
                         sq = __builtin_fmaf(v.x, v.x, sq);
@@ -256,12 +255,15 @@ __device__ __forceinline__ void gemv_body(const uint8_t *__restrict__ w0, const 
                         sq = __builtin_fmaf(v.w, v.w, sq);
                         v = make_float4(g.x * v.x, g.y * v.y, g.z * v.z, g.w * v.w);
                     }
+                    v = make_float4(tlive ? v.x : 0.0f, tlive ? v.y : 0.0f, tlive ? v.z : 0.0f, tlive ? v.w : 0.0f);
                     sum = __builtin_fmaf(q8_s8(qw[c], 0), v.x, sum);
                     sum = __builtin_fmaf(q8_s8(qw[c], 1), v.y, sum);
                     sum = __builtin_fmaf(q8_s8(qw[c], 2), v.z, sum);
                     sum = __builtin_fmaf(q8_s8(qw[c], 3), v.w, sum);
                 }
                 float acc = sum * d;
+                if constexpr (EPI == 1)
+                    sq = tlive ? sq : 0.0f;
                 for (int off = tp >> 1; off >= 1; off >>= 1) {
                     acc += __shfl_xor(acc, off, 64);
                     if constexpr (EPI == 1)

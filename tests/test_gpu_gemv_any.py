@@ -67,3 +67,32 @@ def test_any_cols_infinite_scale(rt):
         assert np.all(np.isinf(y[:, 5])) and np.all(np.isfinite(np.delete(y, 5, axis=1)))
     finally:
         case.close()
+
+
+@pytest.mark.parametrize("cols", [32, 1056, 1536, 4128, 5632])
+def test_any_cols_infinite_norm_weight(rt, cols):
+    """Lanes past the row's last unit, and the threads that take none of the tail's, load unit 0: an
+    infinite norm weight there makes a row infinite (NaN where its quant is 0), as with the norm
+    apart, not NaN from those lanes' 0 * inf. A NaN x there stays its own token's."""
+    case = Case(rt, 64, cols, 4, cols)
+    nw, x = case.nw.copy(), case.x.copy()
+    nw[3], x[2, 5] = np.inf, np.nan
+    rt.to_dev(case.p["nw"], nw)
+    rt.to_dev(case.p["x"], x)
+    try:
+        for kind in ("norm", "pair_norm", "round_norm"):
+            for t in (1, 2, 4):
+                out = []
+                for apart in (False, True):
+                    rt.set_epi_apart(apart)
+                    case.nan()
+                    case.run(kind, 0, t)
+                    out.append([a[:t] for a in case.out()])
+                rt.set_epi_apart(False)
+                for a, b in zip(*out):
+                    assert np.array_equal(np.isnan(a), np.isnan(b)), (kind, t)
+                    assert np.array_equal(a[np.isinf(a)], b[np.isinf(a)]), (kind, t)
+                assert np.isinf(out[1][0][0]).any(), (kind, t)
+    finally:
+        rt.set_epi_apart(False)
+        case.close()
