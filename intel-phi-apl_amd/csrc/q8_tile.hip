@@ -344,6 +344,8 @@ __global__ __launch_bounds__(64 * NW * KG) void gemm_tile(tile_args a)
     auto step = [&](auto Ic) __attribute__((always_inline)) {
         constexpr int I = decltype(Ic)::value, U = 2 * MT;
         constexpr int LP = (SI + TR + U - 3) / (U - 2); /* of the SI + TR groups of loads a unit */
+        constexpr int LW = (SI + LP - 1) / LP;          /* the first unit that loads weights */
+        static_assert(LW + (TR + LP - 1) / LP <= U, "every load of a step is issued in one of its units");
         constexpr int PU = (CP * TR + MT - 1) / MT;                  /* conversion pieces a unit */
         constexpr int VU = (4 * TR + 3 * PU + 3 * TR - 1) / (3 * TR); /* VALU instructions an MFMA */
         const int c = pos[0].c, c1 = clamp(pos[1].c), cn = clamp(pos[NB - 1].c), cw = clamp(pos[WB - 1].c);
@@ -356,12 +358,16 @@ __global__ __launch_bounds__(64 * NW * KG) void gemm_tile(tile_args a)
             const int h = u / MT, m = u % MT;
             if (u + 1 < U)
                 lread(xa[(u + 1) & 1], bufs[I % NB], (u + 1) % MT, (u + 1) / MT);
+            /* in units apart, as no unit's loads move into another (the sched_barrier at its end): the
+             * VN of the next wait counts weights after the last load of the stage */
+            if (u < LW) {
 #pragma unroll
-            for (int k = u * LP; k < (u + 1) * LP; k++) {
-                if (k < SI)
+                for (int k = u * LP; k < (u + 1) * LP && k < SI; k++)
                     stage1(bufs[(I + NB - 1) % NB], cn, k);
-                else if (k < SI + TR)
-                    wload1(W[(I + WB - 1) % WB], cw, k - SI);
+            } else {
+#pragma unroll
+                for (int k = (u - LW) * LP; k < (u - LW + 1) * LP && k < TR; k++)
+                    wload1(W[(I + WB - 1) % WB], cw, k);
             }
             const ops &OC = h ? O1 : O[I & 1];
             f32x4(&r)[TR] = pv[u & 1];
