@@ -31,6 +31,16 @@ __host__ __device__ inline int q8_any_waves(long cols)
     return whole > 0 && whole % 4 == 0 && q8_pow2_from(tail) <= 4 * whole ? whole : whole + 1;
 }
 
+/* The most rows (a round's together, both matrices' of the pair) at which the decode kernels of 5 to 8
+ * waves take an epilogue in at mt tokens. Each workgroup does the norm's arithmetic again, and at 4
+ * tokens an epilogue takes them past 128 registers, which leaves one workgroup a compute unit where
+ * there were two; apart it costs a launch, whatever the rows. Apart against fused, us: the norm on
+ * 8192 columns at 4 tokens at 4096, 8192 and 20480 rows 15.0 / 14.0, 24.0 / 25.8 and 49.8 / 60.7, at
+ * 3 tokens 42.9 / 45.8 at 20480; a round on the norm of 25632 rows at 2 tokens 50.1 / 53.5; the pair on 8192 columns (pair8k: 8 waves of whole 1024s) at 4 tokens
+ * 42.4 / 43.2 at 2 x 8192 rows, 92 / 101 at 2 x 20480; the residual on 5120 columns at 4 tokens 0.97
+ * and 0.84 of fused at 4096 and 20480 rows. */
+inline long q8_epi_rows(int mt, bool pair8k) { return mt == 1 ? 1L << 40 : mt <= 3 || pair8k ? 16384 : 4096; }
+
 /* The decode kernel for cols % 1024 == 0: a workgroup of NW waves owns RW rows and all of K;
  * wave w takes the K-slice [w*1024*S, (w+1)*1024*S), S steps of 64 16-column units (lane l:
  * units l + 64 s). Every load of a lane is issued before any arithmetic, x first and then the

@@ -59,10 +59,14 @@ template <int MT, int PAIR, int EPI>
 static bool any_try(hipStream_t s, const void *w0, const void *w1, long rows, long cols, const float *x, long xs, float *y, const q8_epi &e)
 {
     const int nw = q8_any_waves(cols);
-    int rw = PAIR && MT == 1 ? 4 : 8;
+    /* the pair at 5 to 8 waves from two tokens: 151 to 176 registers at 8 rows leave one workgroup a
+     * compute unit (12288 x 5120 at 3 tokens 45.2 us, 41.1 at 4 rows; four waves and nine or more are 5
+     * to 15 % slower so). Not on the norm at 2 tokens (no gain) and at 4 (10 % slower) */
+    const bool mid = nw > 4 && nw <= 8;
+    int rw = PAIR && (MT == 1 || (mid && (EPI != 1 || MT == 3))) ? 4 : 8;
     while (rw > 2 && rows / rw * nw < (PAIR ? 4096 : 1024))
         rw /= 2;
-    if (cols > 16384 || (EPI == 1 && nw > 8))
+    if (cols > 16384 || (EPI == 1 && nw > 8) || (mid && EPI && (EPI == 1 || MT == 4) && (PAIR + 1) * rows > q8_epi_rows(MT, false)))
         return false;
     if (nw <= 4)
         any_rw<MT, 4, PAIR, EPI>(s, rw, nw, w0, w1, rows, cols, x, xs, y, e);
@@ -104,7 +108,7 @@ static bool round_try(hipStream_t s, const q8_round &r, long cols, const float *
 #define ANY(N)                                                                                                         \
     Q8_LAUNCH(q8_time_name("gemv_round_any", 4, MT, Q8_ROUND_RW, N, EPI), (gemv_round_any<MT, Q8_ROUND_RW, N, EPI>), dim3((unsigned)r.start[r.n]), \
               dim3(64 * nw), s, r, cols, x, xs, e)
-    if (cols > 16384 || nw > (EPI == 1 ? 8 : MT > 2 ? 12 : 16))
+    if (cols > 16384 || nw > (EPI == 1 ? 8 : MT > 2 ? 12 : 16) || (EPI == 1 && nw > 4 && r.start[r.n] * Q8_ROUND_RW > q8_epi_rows(MT, false)))
         return false;
     if (nw <= 4)
         ANY(4);

@@ -274,7 +274,9 @@ void q8_launch_gemv(q8_stream_t stream, const void *w0, const void *w1, long row
 }
 
 /* ---- the epilogue kernels: the layer shapes' K (S = 1 and NW = 2, 4, 6, 12: K = 2048, 4096,
- * 6144, 12288) at 2, 4 or 8 rows a workgroup; other shapes in q8_gemv_any.hip */
+ * 6144, 12288) and 8192, where the instance for any columns takes 132 registers at 4 tokens and this one
+ * fits 128 (the residual 20480 x 8192 59.4 us there, 46.4 here, 47.5 apart), at 2, 4 or 8 rows a
+ * workgroup; other shapes in q8_gemv_any.hip */
 template <int MT, int RW, int PAIR, int EPI>
 static bool gemv_epi_rw(hipStream_t s, int nw, long kb, const uint8_t *a, const uint8_t *b, long rows, long cols, const float *x, long xs, float *y,
                         const q8_epi &e)
@@ -285,7 +287,7 @@ static bool gemv_epi_rw(hipStream_t s, int nw, long kb, const uint8_t *a, const 
                   a, b, rows, cols, x, xs, y, e);                                                                      \
         return true;                                                                                                   \
     }
-    K1(1, 2) K1(1, 4) K1(1, 6)
+    K1(1, 2) K1(1, 4) K1(1, 6) K1(1, 8)
     /* K = 12288 (the down matrix): not the pair (no layer has one there), nor 4 tokens at 8 rows
      * with the norm (both would spill registers) */
     if constexpr (!PAIR && !(MT == 4 && RW == 8 && EPI == 1)) {
@@ -307,6 +309,8 @@ static bool gemv_epi_go(hipStream_t s, const void *w0, const void *w1, long rows
      * round of fewer, longer workgroups) is the faster shape then (12288x4096: 20.5 against 21.3 us) */
     if (PAIR && EPI == 1 && rw == 4 && rows % 8 == 0 && rows / 8 * nw >= 2048)
         rw = 8;
+    if (EPI == 1 && kb == 8 && (PAIR + 1) * rows > q8_epi_rows(MT, PAIR))
+        return false;
     bool done = false;
     if constexpr (EPI == 2 && MT > 1)
         if (rw == 16) { /* K = 12288: 4096 x 12288 with the residual at 4 tokens 18.0 us on 8 rows; 2 us less a layer here */
@@ -459,7 +463,7 @@ static bool round_norm_go(hipStream_t s, int nw, long kb, const q8_round &r, lon
                   cols, x, xs, e);                                                                                     \
         return true;                                                                                                   \
     }
-    K1(1, 2) K1(1, 4) K1(1, 6)
+    K1(1, 2) K1(1, 4) K1(1, 6) K1(1, 8)
     if constexpr (MT < 4) { /* 4 tokens at K = 12288 would spill registers */
         K1(1, 12)
     }
@@ -473,7 +477,7 @@ int q8_launch_gemv_round_epi(q8_stream_t stream, int n, const void *const *w, co
     q8_round r;
     int nw;
     long kb;
-    if (!e.nw || e.res || !round_plan(n, w, rows, cols, t, y, r, nw, kb))
+    if (!e.nw || e.res || !round_plan(n, w, rows, cols, t, y, r, nw, kb) || (kb == 8 && r.start[n] * Q8_ROUND_RW > q8_epi_rows((int)t, false)))
         return -1;
     hipStream_t s = (hipStream_t)stream;
     constexpr int RW = Q8_ROUND_RW;

@@ -96,3 +96,35 @@ def test_any_cols_infinite_norm_weight(rt, cols):
     finally:
         rt.set_epi_apart(False)
         case.close()
+
+
+@pytest.mark.parametrize("rows,cols,kind,t,name", [
+    (1008, 8192, "residual", 4, "gemv_ke<4, 4, 1, 8, 0, 2>"), (1008, 8192, "norm", 3, "gemv_ke<3, 4, 1, 8, 0, 1>"),
+    (4112, 8192, "norm", 4, "gemv_k<4, 8, 1, 8, 0>"), (4096, 8192, "round_norm", 4, "gemv_round<4, 8, 1, 8>"),
+    (4080, 8192, "round_norm", 4, "gemv_round_norm<4, 8, 1, 8>"), (4112, 5152, "norm", 4, "gemv_any<4, 8, 8, 0, 0>"),
+    (4096, 5152, "norm", 4, "gemv_any<4, 8, 8, 0, 1>"), (4112, 5152, "residual", 4, "gemv_any<4, 8, 8, 0, 0>"),
+    (4112, 5152, "residual", 3, "gemv_any<3, 8, 8, 0, 2>"), (4112, 5152, "round_norm", 4, "gemv_round_any<4, 8, 8, 0>"),
+    (6144, 5152, "pair", 3, "gemv_any<3, 4, 8, 1, 0>"), (6144, 5152, "pair_norm", 3, "gemv_any<3, 4, 8, 1, 1>"),
+    (6144, 5152, "pair_norm", 2, "gemv_any<2, 8, 8, 1, 1>"), (2048, 5152, "pair_norm", 4, "gemv_any<4, 2, 8, 1, 1>")])
+def test_five_to_eight_waves(rt, rows, cols, kind, t, name):
+    """The instances that 5 to 8 waves choose at the rows where the rules change: fused up to a few thousand
+    rows, apart above, four rows of the pair; each against the epilogue apart (the residual and the pair
+    the same bits, the norm within its order of summation)."""
+    case = Case(rt, rows, cols, t, rows + cols + t)
+    try:
+        out = []
+        for apart in (False, True):
+            rt.set_epi_apart(apart)
+            case.nan()
+            names = kernels(rt, lambda: case.run(kind, 0, t))
+            if not apart:
+                assert names[0] == name
+            out.append(case.out())
+        for a, b in zip(*out):
+            if "norm" not in kind:
+                assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+            elif not np.isnan(a).all():
+                assert_parity(a, b.astype(np.float64), f"{kind} {rows}x{cols} t={t}")
+    finally:
+        rt.set_epi_apart(False)
+        case.close()
