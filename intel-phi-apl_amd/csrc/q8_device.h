@@ -164,7 +164,8 @@ __device__ __forceinline__ void q8_wave_sums(float (&v)[V], int lane)
     }
 }
 
-/* a + the squares of v's four values, and the norm's sums of W waves (4, or 16, of which the last 8 are zero up to 2048 columns): the pieces of the RMS
+/* a + the squares of v's four values, and the norm's sums of W waves (of 4 up to 1024 columns and of 16
+ * above; W says how many of the first have columns, the others' would add zero): the pieces of the RMS
  * norm's sum, which every kernel that computes the norm apart from a product adds in one order */
 __device__ __forceinline__ float q8_norm_add(float4 v, float a)
 {
@@ -176,13 +177,10 @@ __device__ __forceinline__ float q8_norm_add(float4 v, float a)
 template <int W>
 __device__ __forceinline__ float q8_norm_fold(const float *p)
 {
-    const float a = (p[0] + p[1]) + (p[2] + p[3]);
-    if constexpr (W == 4)
-        return a;
-    else if constexpr (W == 8)
-        return a + ((p[4] + p[5]) + (p[6] + p[7]));
+    if constexpr (W == 1)
+        return p[0];
     else
-        return (a + ((p[4] + p[5]) + (p[6] + p[7]))) + (((p[8] + p[9]) + (p[10] + p[11])) + ((p[12] + p[13]) + (p[14] + p[15])));
+        return q8_norm_fold<W / 2>(p) + q8_norm_fold<W / 2>(p + W / 2);
 }
 
 /* SiLU(g) * u (src/apl/qwen35.apl:38; docs/model.md:29: Sig = 1 / (1 + exp(min(700, -g)))):

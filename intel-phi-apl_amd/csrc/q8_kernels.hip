@@ -352,44 +352,75 @@ int q8_launch_gemv_epi(q8_stream_t stream, const void *w0, const void *w1, long 
     return done ? 0 : -1;
 }
 
-/* The RMS norm apart: one workgroup a token, of 1024 threads above 1024 columns and 256 below; x^2
- * summed by each thread over its columns (4 tid + 4 NT j), then by the wave, and across the waves as
- * q8_norm_fold adds them; xn may be x (xs == cols). A latency chain, not a bandwidth: x and the norm
- * weights are loaded once, up to 16384 columns kept in registers, where 256 threads in four trips
- * that read x again took 4.9 us at 16 tokens of 4096 (traced) against 3.6. */
+/* The RMS norm apart, a workgroup a token. x^2 is summed over the columns of 1024 threads (thread T's are
+ * 4 T + 4096 j, four at a time), then by the wave, and across the 16 waves as q8_norm_fold adds them; up
+ * to 1024 columns the threads are 256. The kernel runs on NT threads, each taking the part of up to Q of
+ * those (T, T + NT, ...; part[] holds the waves' sums either way), so the sums are the same in all of
+ * them; threads without columns only add zeros. xn may be x (xs == cols).
+ *
+ * Few tokens are a latency chain, x and the norm weights loaded at once on 1024 threads: 16 tokens of 4096
+ * columns 3.6 us (traced) against 4.9 on 256. More tokens than compute units are a matter of the
+ * workgroups that a unit holds and of what they keep in registers (the weights are loaded once x^2 is
+ * summed): in a graph 2048 tokens of 1056 columns 4.2 us on 256 threads against 6.8 on 1024, 1024 of 4128
+ * 6.0 on 512 against 6.6, and 4096 of 32 columns 2.8 on 64 against 3.6 on 256. 4 NT S columns stay in
+ * registers between the sum and the scaling, the others are read again. */
 template <int NT, int S>
 __global__ __launch_bounds__(NT) void rmsnorm_k(const float *x, long xs, long cols, const float *__restrict__ nw, float eps, float *xn)
 {
+    constexpr int Q = S < 1024 / NT ? S : 1024 / NT; /* a thread's parts of the 1024 threads, or of those with columns */
+    constexpr bool LATE = NT < 1024 && S > 1;
+    static_assert(S % Q == 0, "a thread's part of column group j is j % Q");
     const float *xr = x + (long)blockIdx.x * xs;
     float *o = xn + (long)blockIdx.x * cols;
+    const long k0 = 4 * (long)threadIdx.x;
     float4 v[S], g[S];
 #pragma unroll
     for (int j = 0; j < S; j++) {
-        const long k = 4 * (long)threadIdx.x + 4L * NT * j, c = k < cols ? k : 0;
-        v[j] = *(const float4 *)(xr + c);
-        g[j] = *(const float4 *)(nw + c);
+        const long k = k0 + 4L * NT * j;
+        if (k < cols) {
+            v[j] = *(const float4 *)(xr + k);
+            if (!LATE)
+                g[j] = *(const float4 *)(nw + k);
+        }
     }
-    float a = 0.0f;
+    float a[Q];
+#pragma unroll
+    for (int q = 0; q < Q; q++)
+        a[q] = 0.0f;
 #pragma unroll
     for (int j = 0; j < S; j++)
-        if (4 * (long)threadIdx.x + 4L * NT * j < cols)
-            a = q8_norm_add(v[j], a);
-    for (long k = 4 * (long)threadIdx.x + 4L * NT * S; k < cols; k += 4 * NT)
-        a = q8_norm_add(*(const float4 *)(xr + k), a);
-    a = q8_wave_sum_dpp(a);
-    __shared__ float part[NT / 64];
-    if ((threadIdx.x & 63) == 0)
-        part[threadIdx.x >> 6] = a;
+        if (k0 + 4L * NT * j < cols)
+            a[j % Q] = q8_norm_add(v[j], a[j % Q]);
+    if constexpr (LATE) {
+#pragma unroll
+        for (int j = 0; j < S; j++) {
+            const long k = k0 + 4L * NT * j;
+            if (k < cols)
+                g[j] = *(const float4 *)(nw + k);
+        }
+    }
+    for (long k = k0 + 4L * NT * S; k < cols; k += 4 * NT * Q)
+#pragma unroll
+        for (int q = 0; q < Q; q++)
+            if (k + 4L * NT * q < cols)
+                a[q] = q8_norm_add(*(const float4 *)(xr + k + 4L * NT * q), a[q]);
+    __shared__ float part[NT / 64 * Q];
+#pragma unroll
+    for (int q = 0; q < Q; q++) {
+        a[q] = q8_wave_sum_dpp(a[q]);
+        if ((threadIdx.x & 63) == 0)
+            part[NT / 64 * q + (threadIdx.x >> 6)] = a[q];
+    }
     __syncthreads();
-    const float sc = 1.0f / sqrtf(eps + q8_norm_fold<NT / 64>(part) / (float)cols);
+    const float sc = 1.0f / sqrtf(eps + q8_norm_fold<NT / 64 * Q>(part) / (float)cols);
     auto put = [&](long k, float4 v, float4 g) { *(float4 *)(o + k) = make_float4(g.x * (v.x * sc), g.y * (v.y * sc), g.z * (v.z * sc), g.w * (v.w * sc)); };
 #pragma unroll
     for (int j = 0; j < S; j++) {
-        const long k = 4 * (long)threadIdx.x + 4L * NT * j;
+        const long k = k0 + 4L * NT * j;
         if (k < cols)
             put(k, v[j], g[j]);
     }
-    for (long k = 4 * (long)threadIdx.x + 4L * NT * S; k < cols; k += 4 * NT)
+    for (long k = k0 + 4L * NT * S; k < cols; k += 4 * NT)
         put(k, *(const float4 *)(xr + k), *(const float4 *)(nw + k));
 }
 
@@ -397,12 +428,24 @@ void q8_launch_rmsnorm(q8_stream_t stream, const float *x, long x_stride, long t
 {
     const hipStream_t s = (hipStream_t)stream;
     const dim3 g((unsigned)t);
-    if (cols <= 1024)
-        rmsnorm_k<256, 1><<<g, dim3(256), 0, s>>>(x, x_stride, cols, nw, eps, xn);
+#define NORM(N, S) rmsnorm_k<N, S><<<g, dim3(N), 0, s>>>(x, x_stride, cols, nw, eps, xn)
+    if (cols <= 256)
+        NORM(64, 1);
+    else if (cols <= 512)
+        NORM(128, 1);
+    else if (cols <= 1024)
+        NORM(256, 1);
+    else if (t > 256 && cols <= 2048)
+        NORM(256, 2);
+    else if (t > 256 && cols <= 4096)
+        NORM(256, 4);
+    else if (t > 256 && cols <= 8192)
+        NORM(512, 4);
     else if (cols <= 4096)
-        rmsnorm_k<1024, 1><<<g, dim3(1024), 0, s>>>(x, x_stride, cols, nw, eps, xn);
+        NORM(1024, 1);
     else
-        rmsnorm_k<1024, 4><<<g, dim3(1024), 0, s>>>(x, x_stride, cols, nw, eps, xn);
+        NORM(1024, 4);
+#undef NORM
 }
 
 __global__ __launch_bounds__(256) void add_k(const float *a, const float *b, long n, float *y)

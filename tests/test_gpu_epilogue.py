@@ -269,3 +269,33 @@ def test_epilogues_random_shapes(rt, oracle, case):
     assert_parity(yn, oracle.gemm_f64d(q8, rows, cols, oracle.rmsnorm_f64(x, nw, EPS)), f"norm product {rows}x{cols} t={t}")
     assert np.array_equal(yr.view(np.uint32), (r + plain).view(np.uint32))
     assert np.array_equal(inplace.view(np.uint32), yr.view(np.uint32))
+
+
+@pytest.mark.parametrize("cols", [4, 32, 256, 260, 512, 516, 1000, 1024, 1028, 2048, 2052, 4096, 4100, 8192, 8196, 12288, 16388, 20480])
+def test_rmsnorm_many_tokens(rt, oracle, cols):
+    """More than 256 tokens run on 256 threads a token: the bits of one token a call (1024 threads), x rows
+    apart and in place, and the F64 norm."""
+    t, xs = 260, cols + 8
+    rng = np.random.default_rng(cols)
+    x = rng.standard_normal((t, xs)).astype(np.float32)
+    nw = (1.0 + 0.1 * rng.standard_normal(cols)).astype(np.float32)
+    dx, dn, do = rt.alloc(x.nbytes), rt.alloc(nw.nbytes), rt.alloc(4 * t * cols)
+    try:
+        rt.to_dev(dx, x)
+        rt.to_dev(dn, nw)
+        many, one, inplace = (np.empty((t, cols), np.float32) for _ in range(3))
+        rt.lib.rt_rmsnorm_dev(rt.R, c.c_void_p(dx), xs, t, cols, c.c_void_p(dn), EPS, c.c_void_p(do))
+        rt.from_dev(many, do)
+        for k in range(t):
+            rt.lib.rt_rmsnorm_dev(rt.R, c.c_void_p(dx + 4 * k * xs), xs, 1, cols, c.c_void_p(dn), EPS, c.c_void_p(do + 4 * k * cols))
+        rt.from_dev(one, do)
+        rt.to_dev(do, np.ascontiguousarray(x[:, :cols]))
+        rt.lib.rt_rmsnorm_dev(rt.R, c.c_void_p(do), cols, t, cols, c.c_void_p(dn), EPS, c.c_void_p(do))
+        rt.from_dev(inplace, do)
+    finally:
+        for p in (dx, dn, do):
+            rt.free(p)
+    assert np.array_equal(many.view(np.uint32), one.view(np.uint32)) and np.array_equal(many.view(np.uint32), inplace.view(np.uint32))
+    ref = oracle.rmsnorm_f64(np.ascontiguousarray(x[:, :cols]), nw, EPS)
+    # cols / 16 additions a wave's chain of 2^-24 each at most, halved by the square root
+    assert np.abs(many - ref).max() <= np.abs(ref).max() * (cols / 16 + 64) * 2.0**-24
