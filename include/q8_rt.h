@@ -169,7 +169,8 @@ void rt_gemv_swiglu_dev(struct rt *R, const void *wg, const void *wu, long rows,
  * norm is s = 1 / sqrt(eps + sum_k x[k]^2 / cols) per token in F32, xn[k] = nw[k] * (x[k] * s); its
  * sum runs in a fixed order for a given shape, so results repeat bit for bit, and a fused and a
  * separate norm differ only by that order (an ulp or so of s). The residual is one F32 add of the
- * product, the same bits fused or apart. */
+ * product, the same bits fused or apart. A y that shares memory with x is allowed with the norm, and
+ * with the residual at t <= 4: the epilogue then runs apart. */
 /* xn = the normed x, t tokens (x rows x_stride floats apart, xn rows cols apart; xn may be x when
  * x_stride == cols); cols % 4 == 0. */
 void rt_rmsnorm_dev(struct rt *R, const float *x, long x_stride, long t, long cols, const float *nw, float eps, float *xn);

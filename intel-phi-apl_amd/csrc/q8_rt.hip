@@ -492,6 +492,13 @@ void kt_cancel(ctx *c)
     c->kt.pop_back();
 }
 
+/* Whether y (n floats) shares memory with x (t rows of cols floats, xs apart): an epilogue in the
+ * product's own launch would read x where other workgroups, or an earlier chunk of tokens, have stored y */
+bool overlaps(const float *x, long xs, long t, long cols, const float *y, long n)
+{
+    return x < y + n && y < x + ((t - 1) * xs + cols);
+}
+
 /* Y = X W^T (or the fused pair) with an epilogue: the RMS norm of x first (e.nw) or the residual
  * added to Y (e.res). Fused into the decode kernel where it takes the shape; else the norm apart
  * into the workspace and then the product, or the residual in the matrix-core product's store, or
@@ -499,7 +506,7 @@ void kt_cancel(ctx *c)
 void product_epi(ctx *c, const void *w0, const void *w1, long rows, long cols, const float *x, long xs, long t, float *y, q8_epi e)
 {
     const q8_stream_t s = (q8_stream_t)c->stream;
-    const bool apart = c->epi_apart != 0;
+    const bool apart = c->epi_apart != 0 || ((e.nw || t <= 4) && overlaps(x, xs, t, cols, y, t * rows));
     if (!c->exact && t <= 4 && !apart) {
         const bool timed = kt_begin(c, RT_K_GEMV + (w1 ? 1 : 0), rows, cols, t);
         if (q8_launch_gemv_epi(s, w0, w1, rows, cols, x, xs, t, y, e) == 0) {
@@ -1160,7 +1167,10 @@ void rt_gemv_round_norm_dev(struct rt *R, int n, const void *const *w, const lon
         check_dev_ptr("rt_gemv_round_norm_dev", y[i], "every y");
     }
     const q8_stream_t s = (q8_stream_t)c->stream;
-    if (!c->exact && t <= 4 && !c->epi_apart) {
+    bool apart = c->epi_apart != 0;
+    for (int i = 0; i < n; i++)
+        apart = apart || overlaps(x, x_stride, t, cols, y[i], t * rows[i]);
+    if (!c->exact && t <= 4 && !apart) {
         long total = 0;
         for (int i = 0; i < n; i++)
             total += rows[i];
@@ -1173,7 +1183,7 @@ void rt_gemv_round_norm_dev(struct rt *R, int n, const void *const *w, const lon
             kt_cancel(c);
     }
     float *xn = reserve_epi(c, (size_t)(t * cols));
-    if (!c->exact && n > 1 && !c->epi_apart && tile_ready(c, n, rows, cols, t, false, true, nullptr)) {
+    if (!c->exact && n > 1 && !apart && tile_ready(c, n, rows, cols, t, false, true, nullptr)) {
         reserve_round(c, n, rows, cols, t);
         long total = 0;
         for (int i = 0; i < n; i++)

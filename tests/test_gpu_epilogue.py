@@ -299,3 +299,40 @@ def test_rmsnorm_many_tokens(rt, oracle, cols):
     ref = oracle.rmsnorm_f64(np.ascontiguousarray(x[:, :cols]), nw, EPS)
     # cols / 16 additions a wave's chain of 2^-24 each at most, halved by the square root
     assert np.abs(many - ref).max() <= np.abs(ref).max() * (cols / 16 + 64) * 2.0**-24
+
+
+@pytest.mark.parametrize("kind,rows,cols,t", [("norm", 1536, 1536, 1), ("norm", 2048, 2048, 4), ("norm", 1056, 1056, 3), ("norm", 4608, 4096, 2816),
+                                              ("norm", 512, 512, 40), ("pair_norm", 1536, 1536, 2), ("round_norm", 1536, 1536, 3), ("round_norm", 2048, 2048, 48),
+                                              ("residual", 1536, 1536, 4), ("residual", 2048, 2048, 1)])
+def test_y_over_x(rt, kind, rows, cols, t):
+    """A y in x's own memory: the epilogue runs apart, bit for bit as apart with a y of its own. 2816 tokens of
+    4096 columns take two limb images, and 4608 rows of the first one's y reach into the second one's x."""
+    rng = np.random.default_rng(rows + t)
+    q8 = synth.q8_rows(rng, rows, cols)
+    w = [rt.upload(q8, rows, cols) for _ in range(2)]
+    x, nw, r = rng.standard_normal((t, cols)).astype(np.float32), _vec(3, cols), rng.standard_normal((t, rows)).astype(np.float32)
+    with Dev(rt) as d:
+        dn, dr, do, dz, shared = d.put(nw), d.put(r), d.empty(4 * t * rows), d.empty(4 * t * rows), d.empty(4 * t * max(rows, cols))
+
+        def run(dy):
+            rt.to_dev(shared, x)
+            p = [c.c_void_p(v) for v in (w[0], w[1], shared, dy, dn, dr)]
+            if kind == "norm":
+                rt.lib.rt_gemm_norm_dev(rt.R, p[0], rows, cols, p[2], cols, t, p[4], EPS, p[3])
+            elif kind == "pair_norm":
+                rt.lib.rt_gemv_swiglu_norm_dev(rt.R, p[0], p[1], rows, cols, p[2], cols, t, p[4], EPS, p[3])
+            elif kind == "residual":
+                rt.lib.rt_gemm_residual_dev(rt.R, p[0], rows, cols, p[2], cols, t, p[5], p[3])
+            else:
+                ws, rr, ys = (c.c_void_p * 2)(w[1], w[0]), (c.c_long * 2)(16, rows), (c.c_void_p * 2)(dz, dy)
+                rt.lib.rt_gemv_round_norm_dev(rt.R, 2, ws, rr, cols, p[2], cols, t, p[4], EPS, ys)
+            return d.get(dy, (t, rows), np.float32)
+
+        rt.set_epi_apart(True)
+        try:
+            want = run(do)
+        finally:
+            rt.set_epi_apart(False)
+        assert np.array_equal(run(shared).view(np.uint32), want.view(np.uint32))
+    for v in w:
+        rt.lib.rt_q8_free(rt.R, c.c_void_p(v))
