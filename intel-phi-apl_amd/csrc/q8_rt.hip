@@ -155,9 +155,6 @@ constexpr size_t KT_MAX = 16384;
  * hundreds of tokens hides behind its arithmetic. Of one size, so that a graph may record any shape
  * once one long product has run. */
 constexpr long TILE_IMG_BYTES = 64L << 20;
-/* Rounds (but those on a norm) run as one launch from 81 tokens, single products and the fused pair
- * from 65: the tests hold the rounds of 17 to 70 tokens to the 64-token round kernels by name. */
-constexpr long TILE_ROUND_MIN = 81;
 
 /* The runtimes alive, in the order rt_init set them up; rt_q8_row takes no struct rt
  * (src/card/rt.h:85) and uses the last of them. */
@@ -574,7 +571,7 @@ bool round_launch(ctx *c, int n, const void *const *w, const long *rows, long co
         /* 64 tokens at a time (a token's bits do not depend on t) */
         float *rp = reserve_round(c, n, rows, cols, t);
         rc = 0;
-        if (t >= TILE_ROUND_MIN && tile_ready(c, n, rows, cols, t, false, false, nullptr)) {
+        if (tile_ready(c, n, rows, cols, t, false, false, nullptr)) {
             tile_run(c, n, w, rows, cols, x, xs, t, y, nullptr, nullptr, nullptr, 0.0f, nullptr);
             launched("the round");
             return true;

@@ -506,38 +506,36 @@ __global__ __launch_bounds__(64 * NW * KG) void gemm_tile(tile_args a)
 
 /* ---------------------------------------------------------------- launchers */
 
-/* The instantiated tiles, as X(MT, RT, NW, NP, NB, KG, us0, us1). For a product (NP 1) 256 rows x 128
- * tokens, 256 x 64, 128 x 64, 64 x 64, 64 x 48 and 64 x 32; for the fused pair 128 rows of both x 128
- * tokens, 128 x 64, 64 x 64 and 64 x 32. The large tile does the most work a limb read and a converted weight; the small ones fill
- * the device where there are few tiles, with two K groups, so that a compute unit still holds 8 (for
- * 64 x 64 4) waves of two row tiles each: one row tile a wave reads 1 KiB of limbs an MFMA, all that
- * LDS gives. 4096 x 12288 at 512 tokens 157 us against 170 for 128 x 64 with one row tile on 8 waves
- * and no K groups; 2048 x 6144 at 203 tokens 55 us against 68 for 64 x 64.
- * A step (one pair of blocks; of both groups' one each) of a round of workgroups takes us0 + us1 f
- * us, f the share of the compute units that hold one (the clock falls as they fill); one workgroup a
- * unit. Measured, 1-6 rounds, f from 1/8 to 1, K = 2048 to 12288: 256 x 128 2.04 at f <= 1/2,
- * 2.3-2.6 at 3/4, 3.1 at 1; 256 x 64 1.25, 1.39, 1.67; 128 x 64 1.53-1.58, 1.56, 1.63-1.80; 64 x 64
- * 1.16-1.22, -, 1.19-1.25; 64 x 48 1.04-1.08; 64 x 32 0.85-0.9, 1.35-1.39 for 1.5 workgroups a unit
- * (two fit); the pair 2.02, 2.42, 2.68; 1.47-1.58 at 3/4, 1.62 at 1; 1.70-1.75; 1.26-1.48. 4096 x 4096 at
- * 144 tokens 34.7 us on 64 x 48 tiles against 40.2 on 64 x 64, 6144 x 2048 at 64 16.6 on 64 x 32 against
- * 21.9. */
+/* The instantiated tiles, as X(MT, RT, NW, NP, NB, KG, ur, us, us2, uf). For a product (NP 1) 256 rows x
+ * 128 tokens, 256 x 64, 128 x 64, 64 x 64, 64 x 48 and 64 x 32; for the fused pair 128 rows of both x 128
+ * tokens, 128 x 64, 64 x 64 and 64 x 32. The large tile does the most work a limb read and a converted
+ * weight; the small ones fill the device where there are few tiles, with two K groups, so that a compute
+ * unit still holds 8 (for 64 x 64 4) waves of two row tiles each: one row tile a wave reads 1 KiB of limbs
+ * an MFMA, all that LDS gives. 4096 x 12288 at 512 tokens 157 us against 170 for 128 x 64 with one row tile
+ * on 8 waves and no K groups; 2048 x 6144 at 203 tokens 55 us against 68 for 64 x 64.
+ *
+ * The costs, in us: a round of workgroups ur, and a step (one pair of blocks; of both groups' one each) us
+ * + uf f, f the workgroups a compute unit of the fullest XCD (the clock falls as they fill). One workgroup
+ * a unit, but where us2 is given, two of which take us2 a step. Fitted to 9331 random calls of 5 to 700
+ * tokens, 64 to 24576 rows and 64 to 14336 columns, each timed on most of its configurations: 80 % of the
+ * times within 7 % (64 x 32: 10 %). */
 #define TILE_CFGS(X)                                                                                                   \
-    X(8, 2, 8, 1, 3, 1, 1.60, 1.20)                                                                                    \
-    X(4, 2, 8, 1, 4, 1, 1.10, 0.45)                                                                                    \
-    X(4, 2, 4, 1, 2, 2, 1.45, 0.27)                                                                                    \
-    X(4, 2, 2, 1, 2, 2, 1.10, 0.12)                                                                                    \
-    X(3, 2, 2, 1, 2, 2, 0.95, 0.08)                                                                                    \
-    X(2, 2, 2, 1, 2, 2, 0.72, 0.14)                                                                                    \
-    X(8, 1, 8, 2, 3, 1, 1.75, 0.90)                                                                                    \
-    X(4, 1, 8, 2, 4, 1, 1.30, 0.30)                                                                                    \
-    X(4, 1, 4, 2, 2, 2, 1.60, 0.15)                                                                                    \
-    X(2, 1, 4, 2, 2, 2, 1.15, 0.30)
+    X(8, 2, 8, 1, 3, 1, 3.48, 1.92, 0, 0.16)                                                                           \
+    X(4, 2, 8, 1, 4, 1, 2.07, 1.22, 0, 0.09)                                                                           \
+    X(4, 2, 4, 1, 2, 2, 1.39, 1.42, 0, 0.04)                                                                           \
+    X(4, 2, 2, 1, 2, 2, 2.00, 1.05, 0, 0.03)                                                                           \
+    X(3, 2, 2, 1, 2, 2, 1.54, 0.91, 0, 0.03)                                                                           \
+    X(2, 2, 2, 1, 2, 2, 0.59, 0.78, 1.15, 0.03)                                                                        \
+    X(8, 1, 8, 2, 3, 1, 3.02, 1.87, 0, 0.29)                                                                           \
+    X(4, 1, 8, 2, 4, 1, 1.96, 1.18, 0, 0.19)                                                                           \
+    X(4, 1, 4, 2, 2, 2, 1.04, 1.42, 0, 0.08)                                                                           \
+    X(2, 1, 4, 2, 2, 2, 0.11, 1.09, 1.91, 0.07)
 
 struct tile_cfg {
     int mt, rt, nw, np, nb, kg;
-    float us0, us1;
+    float ur, us, us2, uf;
 };
-#define CFG(M, R, N, P, B, G, U0, U1) {M, R, N, P, B, G, U0##f, U1##f},
+#define CFG(M, R, N, P, B, G, UR, US, US2, UF) {M, R, N, P, B, G, (float)UR, (float)US, (float)US2, (float)UF},
 static const tile_cfg TILES[] = {TILE_CFGS(CFG)};
 #undef CFG
 
@@ -552,14 +550,14 @@ static long tile_rows(const tile_cfg &k, int n, const long *rows)
 
 static int tile_cus()
 {
-    static int cus = 0;
-    if (!cus) {
-        int dev = 0;
-        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1) {
+    static const int cus = [] {
+        int dev = 0, n = 0;
+        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 8) {
             fprintf(stderr, "q8_tile: the device's compute units are not known\n");
             abort();
         }
-    }
+        return n;
+    }();
     return cus;
 }
 
@@ -579,10 +577,13 @@ static const tile_cfg *tile_plan(int n, const long *rows, long cols, long t, boo
     for (const tile_cfg &k : TILES) {
         if (k.np != (pair ? 2 : 1))
             continue;
-        const long groups = ((t + 15) / 16 + k.mt - 1) / k.mt, wgs = tile_rows(k, n, rows) * groups;
-        const long rounds = (wgs + tile_cus() - 1) / tile_cus();
-        const float step = (float)rounds * (k.us0 + k.us1 * (float)wgs / (float)(rounds * tile_cus()));
-        const float cost = (float)(k.kg == 2 ? half : pairs) * step;
+        /* the kernel gives an XCD every eighth row tile with all its token groups: the fullest one sets the
+         * rounds. 5232 x 4352 at 148 tokens on 82 row tiles of 3 groups puts 33 workgroups on 32 units,
+         * 87 us where 64 x 32 tiles take 49 */
+        const long groups = ((t + 15) / 16 + k.mt - 1) / k.mt, per = (tile_rows(k, n, rows) + 7) / 8 * groups, units = tile_cus() / 8;
+        const long rounds = (per + units - 1) / units;
+        const float step = (k.us2 > 0.0f ? (float)(rounds % 2) * k.us + (float)(rounds / 2) * k.us2 : (float)rounds * k.us) + k.uf * (float)per / (float)units;
+        const float cost = (float)rounds * k.ur + (float)(k.kg == 2 ? half : pairs) * step;
         if (!best || cost < *us) {
             best = &k;
             *us = cost;
@@ -599,8 +600,7 @@ bool q8_tile_takes(int n, const long *rows, long cols, long t, bool pair, bool n
      * a round's many small splits leave the most partials to sum (the 9B DeltaNet quartet at 64
      * tokens: norm, product and sums 59 us, image and tiles 42). Single products and the pair gain
      * nothing (12288 x 4096 at 64 tokens 42 + 3.5 against 35, the pair 61 + 3.5 against 63) */
-    const bool few = t <= 64;
-    if ((few && (t <= 32 || n < 2 || pair || !norm)) || n < 1 || n > Q8_ROUND_MAX || (pair && (n != 2 || rows[0] != rows[1])))
+    if ((t <= 64 && (t <= 32 || n < 2 || pair || !norm)) || n < 1 || n > Q8_ROUND_MAX || (pair && (n != 2 || rows[0] != rows[1])))
         return false;
     /* a row of one block has no two scales to load at once */
     if (cols < 2 * Q8_BLOCK)
@@ -608,24 +608,18 @@ bool q8_tile_takes(int n, const long *rows, long cols, long t, bool pair, bool n
     float us = 0.0f;
     if (!tile_plan(n, rows, cols, t, pair, o, &us))
         return false;
-    float weights = 0.0f, all = 0.0f;
-    for (int i = 0; i < n; i++) {
-        weights += (float)rows[i] * (float)cols;
-        all += (float)rows[i];
-    }
-    /* Against the 64-token launches: measured 35, 34, 20, 21 and 14 us a launch at 12288 x 4096, 4096 x
-     * 12288, 4096 x 4096, 2048 x 6144 and 2048 x 2048 (13 us and 0.44 a million weights; less below
-     * 1024 rows, a few workgroups and their sums: 8 us), a last one of fewer tokens 0.55, 0.7 and 0.85
-     * of that up to 16, 32 and 48; a round 55, 43 and 29 at 50, 42 and 25 million weights (taken as 16 us
-     * and 0.5), its norm 3.5. The image takes 3.5 us, and 0.2 a MiB of it from there (10.5 us at 36
-     * MiB). Few rows leave most of the device idle here, where the 64-token launches split K over it:
-     * 4096 x 12288 at 128 tokens 66 against 117 us. */
-    us += 3.5f + 0.2f * (float)q8_ximage_bytes(t, cols) / 1048576.0f;
-    if (few)
-        return us < (t <= 48 ? 0.85f : 1.0f) * (16.0f + 0.5e-6f * weights) + 3.5f;
-    const long last = t % 64;
-    const float launches = (float)(t / 64) + (last == 0 ? 0.0f : last <= 16 ? 0.55f : last <= 32 ? 0.7f : last <= 48 ? 0.85f : 1.0f);
-    return us < launches * (8.0f + (all < 1024.0f ? all / 1024.0f : 1.0f) * 5.0f + 0.44e-6f * weights);
+    /* and the image's launch, its bytes, the norm in it and the stores, as fitted with TILE_CFGS. Against the
+     * 64-token launches (q8_gemm_us), with 8 % for the error of the two: over 5744 random calls that may
+     * take the tiles, 0.55 of the launches' time in the mean, 5 calls above 1.03 of it and none above
+     * 1.14 (few rows leave most of the device idle here, where the launches split K over it: 1024 x 3072
+     * at 91 tokens 28 against 22.6 us) */
+    long outs = 0;
+    for (int i = 0; i < (pair ? 1 : n); i++)
+        outs += rows[i] * t;
+    us += 5.25f + 0.656f * (float)q8_ximage_bytes(t, cols) / 1048576.0f + 1.1e-6f * (float)outs;
+    if (norm)
+        us += 1.44f + 0.00081f * (float)cols;
+    return 1.08f * us < q8_gemm_us(n, rows, cols, t, norm, o);
 }
 
 void q8_launch_ximage(q8_stream_t stream, const float *x, long x_stride, long t, long cols, const float *nw, float eps, void *img)
@@ -661,7 +655,7 @@ void q8_launch_tile(q8_stream_t stream, int n, const void *const *w, const long 
     const long tiles = tile_rows(*k, n, rows);
     const unsigned grid = (unsigned)((tiles + 7) / 8 * 8 * a.groups);
     bool done = false;
-#define GO(M, R, N, P, B, G, U0, U1)                                                                                \
+#define GO(M, R, N, P, B, G, UR, US, US2, UF)                                                                                \
     if (!done && k->mt == M && k->rt == R && k->nw == N && k->np == P && k->kg == G) {                                 \
         Q8_LAUNCH(q8_time_name("gemm_tile", 6, M, R, N, P, B, G), (gemm_tile<M, R, N, P, B, G>), dim3(grid), dim3(64 * N * G), s, a); \
         done = true;                                                                                                   \

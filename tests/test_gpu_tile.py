@@ -114,6 +114,7 @@ def test_long_prompt_bits(rt, rows, cols, t, ks):
         for kind in KINDS:
             name, one, parts = case.whole_and_parts(kind)
             print("long prompt", rows, cols, t, ks, kind, name, flush=True)
+            assert name.startswith("gemm_tile<"), kind
             for a, b in zip(one, parts):
                 assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), kind
     finally:
@@ -121,26 +122,35 @@ def test_long_prompt_bits(rt, rows, cols, t, ks):
         case.close()
 
 
-def test_every_tile_runs_and_few_rows_do_not(rt):
-    """The configurations the rule chooses over sizes (each at least once), and matrices
-    of few rows on the 64-token launches, which split K over the device."""
-    seen = set()
-    for rows, cols, t in [(256, 64, 300), (4096, 1024, 512), (4096, 1024, 1024), (4096, 1024, 2048), (12288, 256, 512), (16384, 256, 1024), (2048, 512, 130), (4096, 1024, 144), (2048, 1024, 200),
-                          (1024, 512, 66), (4096, 512, 200)]:
-        case = Case(rt, rows, cols, t, 3)
-        try:
-            for kind in ("product", "pair"):
-                seen |= set(kernels(rt, lambda: case.run(kind, 0, t)))
-        finally:
-            case.close()
-    print(sorted(seen), flush=True)
-    assert {n for n in seen if n.startswith("gemm_tile<")} >= {f"gemm_tile<{v}>" for v in ("8, 2, 8, 1, 3, 1", "4, 2, 8, 1, 4, 1", "4, 2, 4, 1, 2, 2",
-                                                                                      "4, 2, 2, 1, 2, 2", "8, 1, 8, 2, 3, 1", "4, 1, 8, 2, 4, 1",
-                                                                                      "4, 1, 4, 2, 2, 2", "3, 2, 2, 1, 2, 2", "2, 2, 2, 1, 2, 2",
-                                                                                      "2, 1, 4, 2, 2, 2")}
-    case = Case(rt, 16, 8192, 200, 4)
+# each configuration, at several K splits of odd block counts, with partial tiles of rows and tokens
+TILES = [("8, 2, 8, 1, 3, 1", 12304, 736, 260), ("4, 2, 8, 1, 4, 1", 10256, 736, 130), ("4, 2, 4, 1, 2, 2", 11280, 736, 66), ("4, 2, 2, 1, 2, 2", 5136, 736, 97),
+         ("3, 2, 2, 1, 2, 2", 528, 736, 560), ("2, 2, 2, 1, 2, 2", 240, 736, 66), ("8, 1, 8, 2, 3, 1", 11280, 736, 130), ("4, 1, 8, 2, 4, 1", 11280, 736, 66),
+         ("4, 1, 4, 2, 2, 2", 528, 736, 513), ("2, 1, 4, 2, 2, 2", 240, 736, 66)]
+
+
+@pytest.mark.parametrize("tile,rows,cols,t", TILES)
+def test_every_tile_bits(rt, tile, rows, cols, t):
+    """Every configuration by name, where the rule chooses it, bit for bit the 64-token launches."""
+    case = Case(rt, rows, cols, t, rows + t)
     try:
-        assert kernels(rt, lambda: case.run("product", 0, 200))[0].startswith("gemm_mfma<")
+        name, one, parts = case.whole_and_parts("pair" if tile.split(", ")[3] == "2" else "product")
+        assert name == f"gemm_tile<{tile}>"
+        assert np.array_equal(one[0].view(np.uint32), parts[0].view(np.uint32))
+    finally:
+        case.close()
+
+
+@pytest.mark.parametrize("kind,rows,cols,t,name", [
+    ("product", 5232, 4352, 148, "gemm_tile<2, 2, 2, 1, 2, 2>"), ("product", 1024, 3072, 91, "gemm_mfma<"), ("product", 16, 8192, 200, "gemm_mfma<"),
+    ("norm", 5376, 3040, 116, "gemm_tile<4, 2, 2, 1, 2, 2>"), ("round_norm", 256, 1984, 60, "gemm_mfma_round<"), ("round_norm", 2480, 3072, 53, "gemm_mfma_round<"),
+    ("round_norm", 12288, 4096, 64, "gemm_tile<"), ("round", 8192, 4096, 65, "gemm_tile<"), ("round", 256, 4096, 65, "gemm_mfma_round<")])
+def test_the_rule(rt, kind, rows, cols, t, name):
+    """Sizes at which another route was up to 1.9 times slower: tiles whose row tiles and token groups fill one
+    XCD past its compute units, few rows (the 64-token launches split K over the device), and rounds of 65
+    tokens."""
+    case = Case(rt, rows, cols, t, 3)
+    try:
+        assert kernels(rt, lambda: case.run(kind, 0, t))[0].startswith(name)
     finally:
         case.close()
 
@@ -258,3 +268,41 @@ def test_round_on_a_norm_up_to_64_tokens(rt, rows, cols, t):
     finally:
         rt.set_epi_apart(False)
         case.close()
+
+
+@pytest.mark.parametrize("t", [65, 68, 70])
+@pytest.mark.parametrize("shapes", [[8192, 1024, 1024], [2048, 2048]], ids=["qkv", "pair"])
+def test_rounds_of_64_tokens_and_a_rest(q8rt, rt, t, shapes):
+    """The 64-token round and one of the last 1, 4 and 6 tokens, as a runtime without a limb image records
+    them: the bits of the tiles' round."""
+    rng = np.random.default_rng(t)
+    q8, x, n = [synth.q8_rows(rng, r, 4096) for r in shapes], synth.x_f32(rng, t, 4096), len(shapes)
+
+    def run(r, record):
+        w = [r.upload(q, k, 4096) for q, k in zip(q8, shapes)]
+        px, py = r.alloc(x.nbytes), [r.alloc(4 * t * k) for k in shapes]
+        r.to_dev(px, x)
+        args = (r.R, n, (P * n)(*w), (c.c_long * n)(*shapes), 4096, P(px), 4096)
+        if record:
+            r.lib.rt_gemv_round_dev(*args, 64, (P * n)(*py))  # the rounds' workspace
+            r.lib.rt_graph_begin(r.R)
+        r.lib.rt_gemv_round_dev(*args, t, (P * n)(*py))
+        if record:
+            g = P(r.lib.rt_graph_end(r.R))
+            r.lib.rt_graph_launch(r.R, g)
+            r.lib.rt_graph_launch(r.R, g)
+        out = [np.empty((t, k), np.float32) for k in shapes]
+        for a, p in zip(out, py):
+            r.from_dev(a, p)
+        if record:
+            r.lib.rt_graph_free(r.R, g)
+        for p in (px, *py):
+            r.free(p)
+        for v in w:
+            r.lib.rt_q8_free(r.R, P(v))
+        return out
+
+    assert kernels(rt, lambda: run(rt, False))[0].startswith("gemm_tile<")
+    with q8rt.Runtime() as r2:
+        for a, b in zip(run(rt, False), run(r2, True)):
+            assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
