@@ -712,9 +712,12 @@ __global__ __launch_bounds__(64 * NW) void read_xres(const uint8_t *w, long rows
 /* The sum of an output's ks partials (splits step floats apart), in split order: sixteen splits' loads
  * in flight at a time, all issued before the first add (past the last split the index is clamped and
  * the value not added). V: an output a thread (float), or four neighbouring ones (float4; rows are
- * whole 16s) where that still gives every compute unit a workgroup, sum_vec: at 64 tokens the round
- * of 12320 rows (33 MB of partials) 9.3 us against 9.9 with one, the 12288-row pair 7.1 against 8.3;
- * at 10 tokens of 7120 rows four a thread were 0.7 us slower. */
+ * whole 16s) where that still gives every compute unit three workgroups, sum_vec: at 64 tokens the round
+ * of 12320 rows (33 MB of partials) 9.3 us against 9.9 with one, the 12288-row pair 7.1 against 8.3, the
+ * product 16384 x 4096 with its sums 42.0 against 43.5. On fewer outputs, a last workgroup on some units
+ * alone, and where a product has more than 32 splits (few rows of many columns, each thread's chain of
+ * adds four times as wide), one a thread is the faster: the round 4096 + 32 + 32 rows of 10240 columns at
+ * 64 tokens 42.4 us against 46.3, 12288 + 32 + 32 87.3 against 89.8. */
 __device__ __forceinline__ float4 sum_add(float4 a, float4 b) { return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w); }
 __device__ __forceinline__ float sum_add(float a, float b) { return a + b; }
 __device__ __forceinline__ float4 sum_swiglu(float4 g, float4 u)
@@ -739,8 +742,8 @@ __device__ __forceinline__ V split_sum(const float *__restrict__ part, int ks, l
     return v;
 }
 /* the outputs a thread of a sum of n outputs, and its grid */
-static bool sum_vec(long n) { return n >= 4L * 256 * 256; }
-static dim3 sum_grid(long n) { return dim3((unsigned)(((sum_vec(n) ? n / 4 : n) + 255) / 256)); }
+static bool sum_vec(long n, int ks) { return n >= 3L * 4 * 256 * 256 && ks <= 32; }
+static dim3 sum_grid(long n, bool vec) { return dim3((unsigned)(((vec ? n / 4 : n) + 255) / 256)); }
 template <class V>
 __device__ __forceinline__ long sum_first()
 {
@@ -1136,16 +1139,21 @@ int q8_launch_gemm_round(q8_stream_t stream, int n, const void *const *w, const 
     const long tp = (t + 15) / 16 * 16;
     if (pair_y) {
         const long outs = all.ostart[1];
-        if (sum_vec(outs))
-            gemm_swiglu_round<float4><<<sum_grid(outs), dim3(256), 0, s>>>(all, tp, pair_y);
+        const bool vec = sum_vec(outs, all.ks[0]);
+        if (vec)
+            gemm_swiglu_round<float4><<<sum_grid(outs, vec), dim3(256), 0, s>>>(all, tp, pair_y);
         else
-            gemm_swiglu_round<float><<<sum_grid(outs), dim3(256), 0, s>>>(all, tp, pair_y);
+            gemm_swiglu_round<float><<<sum_grid(outs, vec), dim3(256), 0, s>>>(all, tp, pair_y);
     } else if (parts > 0) {
         const long outs = all.ostart[n];
-        if (sum_vec(outs))
-            gemm_sum_round<float4><<<sum_grid(outs), dim3(256), 0, s>>>(all, tp);
+        int ks = 1;
+        for (int p = 0; p < n; p++)
+            ks = all.ks[p] > ks ? all.ks[p] : ks;
+        const bool vec = sum_vec(outs, ks);
+        if (vec)
+            gemm_sum_round<float4><<<sum_grid(outs, vec), dim3(256), 0, s>>>(all, tp);
         else
-            gemm_sum_round<float><<<sum_grid(outs), dim3(256), 0, s>>>(all, tp);
+            gemm_sum_round<float><<<sum_grid(outs, vec), dim3(256), 0, s>>>(all, tp);
     }
     return 0;
 }
@@ -1210,9 +1218,10 @@ void q8_launch_gemm_mfma(q8_stream_t stream, const void *w, long rows, long cols
         abort();
     }
     if (ks > 1) {
-        if (sum_vec(t * rows))
-            gemm_sum<float4><<<sum_grid(t * rows), dim3(256), 0, s>>>(part, ks, t, (t + 15) / 16 * 16, rows, y, res);
+        const bool vec = sum_vec(t * rows, ks);
+        if (vec)
+            gemm_sum<float4><<<sum_grid(t * rows, vec), dim3(256), 0, s>>>(part, ks, t, (t + 15) / 16 * 16, rows, y, res);
         else
-            gemm_sum<float><<<sum_grid(t * rows), dim3(256), 0, s>>>(part, ks, t, (t + 15) / 16 * 16, rows, y, res);
+            gemm_sum<float><<<sum_grid(t * rows, vec), dim3(256), 0, s>>>(part, ks, t, (t + 15) / 16 * 16, rows, y, res);
     }
 }

@@ -306,3 +306,29 @@ def test_rounds_of_64_tokens_and_a_rest(q8rt, rt, t, shapes):
     with q8rt.Runtime() as r2:
         for a, b in zip(run(rt, False), run(r2, True)):
             assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+
+
+@pytest.mark.parametrize("cols", [1024, 3104])
+def test_round_sums_of_many_outputs(rt, cols):
+    """A round of 788480 outputs at 64 tokens sums four outputs a thread where its products have at most 32
+    splits (1024 columns), and one where its 32 rows have 49 (3104): each product's bits are its own
+    launch's."""
+    t, shapes = 64, [12288, 32]
+    rng = np.random.default_rng(cols)
+    q8, x = [synth.q8_rows(rng, r, cols) for r in shapes], synth.x_f32(rng, t, cols)
+    w = [rt.upload(q, r, cols) for q, r in zip(q8, shapes)]
+    px, py, pz = rt.alloc(x.nbytes), [rt.alloc(4 * t * r) for r in shapes], [rt.alloc(4 * t * r) for r in shapes]
+    try:
+        rt.to_dev(px, x)
+        rt.lib.rt_gemv_round_dev(rt.R, 2, (P * 2)(*w), (c.c_long * 2)(*shapes), cols, P(px), cols, t, (P * 2)(*py))
+        for v, r, a, b in zip(w, shapes, py, pz):
+            rt.lib.rt_gemm_dev(rt.R, P(v), r, cols, P(px), cols, t, P(b))
+            one, two = np.empty((t, r), np.float32), np.empty((t, r), np.float32)
+            rt.from_dev(one, a)
+            rt.from_dev(two, b)
+            assert np.array_equal(one.view(np.uint32), two.view(np.uint32)), r
+    finally:
+        for p in (px, *py, *pz):
+            rt.free(p)
+        for v in w:
+            rt.lib.rt_q8_free(rt.R, P(v))
