@@ -308,10 +308,10 @@ long q8_gemm_round_part_floats(int n, const long *rows, long cols, long t, q8_ge
 #define Q8_SPLIT_PAIRS 2
 void q8_gemm_split(long rows, long cols, q8_gemm_opts o, int *ks, int *cps);
 /* The time in us of n products of one x (n == 2 of a shape: also the fused pair) at t tokens as 64-token
- * launches with their sums, and of the norm before them, from the sizes alone. Fitted to 9331 random
- * calls of 5 to 700 tokens, 64 to 24576 rows and 64 to 14336 columns: 80 % of those above 32 tokens
- * within 10 %. */
-float q8_gemm_us(int n, const long *rows, long cols, long t, bool norm, q8_gemm_opts o);
+ * launches with their sums (*sums: the part of the partials' stores and sums), and of the norm before
+ * them, from the sizes alone. Fitted to 12615 random
+ * calls of 33 to 700 tokens, 64 to 24576 rows and 64 to 14336 columns: 80 % of them within 8 %. */
+float q8_gemm_us(int n, const long *rows, long cols, long t, bool norm, q8_gemm_opts o, float *sums);
 /* More than 64 tokens (rounds on a norm more than 32) as one launch (q8_tile.hip): whether it takes n
  * products sharing x (pair: the fused pair, n == 2 of one shape; norm: on the RMS norm of x, which the
  * image then holds) and is the faster route, from their sizes alone. Then the limb

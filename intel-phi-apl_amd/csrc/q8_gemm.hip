@@ -933,28 +933,28 @@ static gemm_plan plan_of(long rows, long cols, long t, q8_gemm_opts o)
 
 void q8_gemm_split(long rows, long cols, q8_gemm_opts o, int *ks, int *cps) { split_of(rows, cols, nw_of(rows, cols, o.ks), o.ks, ks, cps); }
 
-float q8_gemm_us(int n, const long *rows, long cols, long t, bool norm, q8_gemm_opts o)
+float q8_gemm_us(int n, const long *rows, long cols, long t, bool norm, q8_gemm_opts o, float *sums)
 {
-    /* a launch of 1 to 4 token tiles, and of 3 or 4 as a pair: base, then a range of the longest chain
-     * of them (rounds of workgroups times the ranges of a split) by the share of 16 waves and apart from
-     * it, and a range of 16 waves a compute unit */
+    /* a launch of 1 to 4 token tiles, and of 3 or 4 as a pair: base, then a range of the chain (the longest
+     * split of each round of workgroups) by the share of 16 waves and apart from it, and a range of 16
+     * waves a compute unit */
     struct launch {
         float base, waves, chain, work;
     };
-    static const launch LAUNCH[6] = {{3.78f, 0.96f, 0.0f, 0.64f}, {2.44f, 0.0f, 0.81f, 0.80f}, {2.91f, 1.34f, 0.76f, 0.76f},
-                                     {3.34f, 0.91f, 1.65f, 0.57f}, {5.28f, 0.0f, 3.20f, 0.51f}, {4.17f, 0.0f, 4.77f, 0.0f}};
+    static const launch LAUNCH[6] = {{3.76f, 1.25f, 0.0f, 0.42f}, {2.66f, 0.0f, 0.83f, 0.83f}, {3.31f, 1.20f, 0.76f, 0.95f},
+                                     {3.78f, 0.74f, 1.64f, 0.87f}, {6.70f, 0.0f, 2.97f, 1.47f}, {5.92f, 0.0f, 4.43f, 1.17f}};
     gemm_plan pl[Q8_ROUND_MAX];
     long all = 0;
-    int big = 0, ks = 1, cps = 1;
+    int big = 0, ks = 1;
     for (int i = 0; i < n; i++) {
         pl[i] = plan_of(rows[i], cols, 64, o);
         all += rows[i];
         big = rows[i] > rows[big] ? i : big;
         ks = pl[i].ks > ks ? pl[i].ks : ks;
-        cps = pl[i].cps > cps ? pl[i].cps : cps;
     }
     const long units = resident_xres(16);
-    float us = (norm ? 2.6f + 2.0e-6f * (float)t * (float)cols : 0.0f) + 0.84e-6f * (float)all * (float)t;
+    *sums = 0.0f;
+    float us = (norm ? 2.46f + 2.69e-6f * (float)t * (float)cols : 0.0f) + 0.88e-6f * (float)all * (float)t;
     for (int last = 0; last < 2; last++) { /* the 64-token launches, and the one of the rest */
         const long count = last ? t % 64 > 0 : t / 64;
         const int mt = last ? (int)((t % 64 + 15) / 16) : 4;
@@ -963,23 +963,33 @@ float q8_gemm_us(int n, const long *rows, long cols, long t, bool norm, q8_gemm_
         const int nw = mt == 2 ? 8 : pl[big].c.nw;
         const bool two = n == 2 && rows[0] == rows[1] && mt >= 3 && nw == 12;
         const launch &l = LAUNCH[two ? mt + 1 : mt - 1];
-        long wgs = 0, ranges = 0;
+        long wgs = 0, ranges = 0, chain = 0, longest = 0; /* longest: of the round that workgroup wgs is in */
         float parts = 0.0f;
         for (int i = 0; i < n; i++) {
-            const long w = (rows[i] + 16L * nw - 1) / (16L * nw) * pl[i].ks;
-            if (!two || i == 0) {
-                wgs += w;
-                ranges += w * pl[i].cps;
-            }
             if (pl[i].ks > 1)
                 parts += (float)pl[i].ks * (float)(16 * mt) * (float)rows[i];
+            if (two && i > 0)
+                continue;
+            const long w = (rows[i] + 16L * nw - 1) / (16L * nw) * pl[i].ks, cps = pl[i].cps;
+            const long left = (units - wgs % units) % units; /* places left in the round begun */
+            if (left > 0 && cps > longest) {
+                chain += cps - longest;
+                longest = cps;
+            }
+            if (w > left) {
+                chain += (w - left + units - 1) / units * cps;
+                longest = cps;
+            }
+            wgs += w;
+            ranges += w * cps;
         }
-        float chain = (float)((wgs + units - 1) / units) * (float)ranges / (float)wgs;
-        chain = chain > (float)cps ? chain : (float)cps;
         const float share = (float)nw / 16.0f;
-        float one = l.base + (l.waves * share + l.chain) * chain + l.work * (float)ranges * share / (float)units;
-        one += (ks > 1 ? 2.76f : 0.0f) + 1.78e-6f * parts + (n > 1 ? 0.91f : 0.0f) + 0.91f * (float)((ks + 15) / 16);
-        us += (float)count * one;
+        const float stream = l.base + (l.waves * share + l.chain) * (float)chain + l.work * (float)ranges * share / (float)units;
+        float sum = (ks > 1 ? 2.96f : 0.0f) + 1.23e-6f * parts + 0.84f * (float)((ks + 15) / 16);
+        if (n > 1 && !two)
+            sum += 0.45f + 0.76e-6f * parts;
+        us += (float)count * (stream + sum);
+        *sums += (float)count * sum;
     }
     return us;
 }

@@ -506,7 +506,7 @@ __global__ __launch_bounds__(64 * NW * KG) void gemm_tile(tile_args a)
 
 /* ---------------------------------------------------------------- launchers */
 
-/* The instantiated tiles, as X(MT, RT, NW, NP, NB, KG, ur, us, us2, uf). For a product (NP 1) 256 rows x
+/* The instantiated tiles, as X(MT, RT, NW, NP, NB, KG, ur, us, us2, uf, uh). For a product (NP 1) 256 rows x
  * 128 tokens, 256 x 64, 128 x 64, 64 x 64, 64 x 48 and 64 x 32; for the fused pair 128 rows of both x 128
  * tokens, 128 x 64, 64 x 64 and 64 x 32. The large tile does the most work a limb read and a converted
  * weight; the small ones fill the device where there are few tiles, with two K groups, so that a compute
@@ -516,26 +516,28 @@ __global__ __launch_bounds__(64 * NW * KG) void gemm_tile(tile_args a)
  *
  * The costs, in us: a round of workgroups ur, and a step (one pair of blocks; of both groups' one each) us
  * + uf f, f the workgroups a compute unit of the fullest XCD (the clock falls as they fill). One workgroup
- * a unit, but where us2 is given, two of which take us2 a step. Fitted to 9331 random calls of 5 to 700
+ * a unit, but where us2 is given, two of which take us2 a step. Token groups share a row tile's weights
+ * in their XCD's L2, and one group alone loads them from HBM: with g groups all of it times 1 + uh f / g^2
+ * (f up to 1; with us2 from 1/2 to 2, as f - 1/2). Fitted to 14488 random calls of 5 to 700
  * tokens, 64 to 24576 rows and 64 to 14336 columns, each timed on most of its configurations: 80 % of the
  * times within 7 % (64 x 32: 10 %). */
 #define TILE_CFGS(X)                                                                                                   \
-    X(8, 2, 8, 1, 3, 1, 3.48, 1.92, 0, 0.16)                                                                           \
-    X(4, 2, 8, 1, 4, 1, 2.07, 1.22, 0, 0.09)                                                                           \
-    X(4, 2, 4, 1, 2, 2, 1.39, 1.42, 0, 0.04)                                                                           \
-    X(4, 2, 2, 1, 2, 2, 2.00, 1.05, 0, 0.03)                                                                           \
-    X(3, 2, 2, 1, 2, 2, 1.54, 0.91, 0, 0.03)                                                                           \
-    X(2, 2, 2, 1, 2, 2, 0.59, 0.78, 1.15, 0.03)                                                                        \
-    X(8, 1, 8, 2, 3, 1, 3.02, 1.87, 0, 0.29)                                                                           \
-    X(4, 1, 8, 2, 4, 1, 1.96, 1.18, 0, 0.19)                                                                           \
-    X(4, 1, 4, 2, 2, 2, 1.04, 1.42, 0, 0.08)                                                                           \
-    X(2, 1, 4, 2, 2, 2, 0.11, 1.09, 1.91, 0.07)
+    X(8, 2, 8, 1, 3, 1, 3.48, 1.92, 0, 0.16, 0.12)                                                                           \
+    X(4, 2, 8, 1, 4, 1, 2.07, 1.22, 0, 0.09, 0.16)                                                                           \
+    X(4, 2, 4, 1, 2, 2, 1.39, 1.42, 0, 0.04, 0.18)                                                                           \
+    X(4, 2, 2, 1, 2, 2, 2.00, 1.05, 0, 0.03, 0.08)                                                                           \
+    X(3, 2, 2, 1, 2, 2, 1.54, 0.91, 0, 0.03, 0.10)                                                                           \
+    X(2, 2, 2, 1, 2, 2, 0.59, 0.78, 1.15, 0.03, 0.40)                                                                        \
+    X(8, 1, 8, 2, 3, 1, 3.02, 1.87, 0, 0.29, 0.00)                                                                           \
+    X(4, 1, 8, 2, 4, 1, 1.96, 1.18, 0, 0.19, 0.16)                                                                           \
+    X(4, 1, 4, 2, 2, 2, 1.04, 1.42, 0, 0.08, 0.15)                                                                           \
+    X(2, 1, 4, 2, 2, 2, 0.11, 1.09, 1.91, 0.07, 0.40)
 
 struct tile_cfg {
     int mt, rt, nw, np, nb, kg;
-    float ur, us, us2, uf;
+    float ur, us, us2, uf, uh;
 };
-#define CFG(M, R, N, P, B, G, UR, US, US2, UF) {M, R, N, P, B, G, (float)UR, (float)US, (float)US2, (float)UF},
+#define CFG(M, R, N, P, B, G, UR, US, US2, UF, UH) {M, R, N, P, B, G, (float)UR, (float)US, (float)US2, (float)UF, (float)UH},
 static const tile_cfg TILES[] = {TILE_CFGS(CFG)};
 #undef CFG
 
@@ -582,8 +584,10 @@ static const tile_cfg *tile_plan(int n, const long *rows, long cols, long t, boo
          * 87 us where 64 x 32 tiles take 49 */
         const long groups = ((t + 15) / 16 + k.mt - 1) / k.mt, per = (tile_rows(k, n, rows) + 7) / 8 * groups, units = tile_cus() / 8;
         const long rounds = (per + units - 1) / units;
-        const float step = (k.us2 > 0.0f ? (float)(rounds % 2) * k.us + (float)(rounds / 2) * k.us2 : (float)rounds * k.us) + k.uf * (float)per / (float)units;
-        const float cost = (float)rounds * k.ur + (float)(k.kg == 2 ? half : pairs) * step;
+        const float f = (float)per / (float)units;
+        const float step = (k.us2 > 0.0f ? (float)(rounds % 2) * k.us + (float)(rounds / 2) * k.us2 : (float)rounds * k.us) + k.uf * f;
+        const float fill = k.us2 > 0.0f ? (f < 0.5f ? 0.0f : f < 2.0f ? f - 0.5f : 1.5f) : f < 1.0f ? f : 1.0f;
+        const float cost = ((float)rounds * k.ur + (float)(k.kg == 2 ? half : pairs) * step) * (1.0f + k.uh * fill / (float)(groups * groups));
         if (!best || cost < *us) {
             best = &k;
             *us = cost;
@@ -608,18 +612,27 @@ bool q8_tile_takes(int n, const long *rows, long cols, long t, bool pair, bool n
     float us = 0.0f;
     if (!tile_plan(n, rows, cols, t, pair, o, &us))
         return false;
-    /* and the image's launch, its bytes, the norm in it and the stores, as fitted with TILE_CFGS. Against the
-     * 64-token launches (q8_gemm_us), with 8 % for the error of the two: over 5744 random calls that may
-     * take the tiles, 0.55 of the launches' time in the mean, 5 calls above 1.03 of it and none above
-     * 1.14 (few rows leave most of the device idle here, where the launches split K over it: 1024 x 3072
-     * at 91 tokens 28 against 22.6 us) */
+    /* and the image's launch, its bytes, the norm in it and the stores, as fitted with TILE_CFGS, against the
+     * 64-token launches (q8_gemm_us). Above 64 tokens 8 % ahead, for the error of the two: of 8311 random
+     * calls there 8 took more than 1.03 of the launches' time (few rows leave most of the device idle
+     * here, where the launches split K over it: 1024 x 3072 at 91 tokens 28 against 22.6 us; below 512 rows
+     * 20 %, 256 x 1504 at 94 tokens 17.2 against 15.7 and priced 9 % below). Up to 64
+     * tokens the streams' errors weigh more, large matrices' above all (13568 + 1696 + 32 rows of 3136
+     * columns at 53 tokens 54.5 against 50.9 us, priced 5 % below): 20 % ahead above 36 million weights and
+     * 3 % below, and no lead where 40 % of the launches' time is their partials and sums, which the tiles
+     * do without (the 9B DeltaNet quartet at 64 tokens 55.9 against 58.9 us) */
     long outs = 0;
     for (int i = 0; i < (pair ? 1 : n); i++)
         outs += rows[i] * t;
     us += 5.25f + 0.656f * (float)q8_ximage_bytes(t, cols) / 1048576.0f + 1.1e-6f * (float)outs;
     if (norm)
         us += 1.44f + 0.00081f * (float)cols;
-    return 1.08f * us < q8_gemm_us(n, rows, cols, t, norm, o);
+    float sums = 0.0f, weights = 0.0f;
+    for (int i = 0; i < n; i++)
+        weights += (float)rows[i] * (float)cols;
+    const float launches = q8_gemm_us(n, rows, cols, t, norm, o, &sums);
+    const float lead = t > 64 ? (weights < 512.0f * (float)cols ? 1.2f : 1.08f) : sums >= 0.4f * launches ? 1.0f : weights > 36e6f ? 1.2f : 1.03f;
+    return lead * us < launches;
 }
 
 void q8_launch_ximage(q8_stream_t stream, const float *x, long x_stride, long t, long cols, const float *nw, float eps, void *img)
@@ -655,7 +668,7 @@ void q8_launch_tile(q8_stream_t stream, int n, const void *const *w, const long 
     const long tiles = tile_rows(*k, n, rows);
     const unsigned grid = (unsigned)((tiles + 7) / 8 * 8 * a.groups);
     bool done = false;
-#define GO(M, R, N, P, B, G, UR, US, US2, UF)                                                                                \
+#define GO(M, R, N, P, B, G, UR, US, US2, UF, UH)                                                                              \
     if (!done && k->mt == M && k->rt == R && k->nw == N && k->np == P && k->kg == G) {                                 \
         Q8_LAUNCH(q8_time_name("gemm_tile", 6, M, R, N, P, B, G), (gemm_tile<M, R, N, P, B, G>), dim3(grid), dim3(64 * N * G), s, a); \
         done = true;                                                                                                   \

@@ -123,7 +123,7 @@ def test_long_prompt_bits(rt, rows, cols, t, ks):
 
 
 # each configuration, at several K splits of odd block counts, with partial tiles of rows and tokens
-TILES = [("8, 2, 8, 1, 3, 1", 12304, 736, 260), ("4, 2, 8, 1, 4, 1", 10256, 736, 130), ("4, 2, 4, 1, 2, 2", 11280, 736, 66), ("4, 2, 2, 1, 2, 2", 5136, 736, 97),
+TILES = [("8, 2, 8, 1, 3, 1", 12304, 736, 260), ("4, 2, 8, 1, 4, 1", 10256, 736, 130), ("4, 2, 4, 1, 2, 2", 11280, 736, 66), ("4, 2, 2, 1, 2, 2", 1040, 736, 513),
          ("3, 2, 2, 1, 2, 2", 528, 736, 560), ("2, 2, 2, 1, 2, 2", 240, 736, 66), ("8, 1, 8, 2, 3, 1", 11280, 736, 130), ("4, 1, 8, 2, 4, 1", 11280, 736, 66),
          ("4, 1, 4, 2, 2, 2", 528, 736, 513), ("2, 1, 4, 2, 2, 2", 240, 736, 66)]
 
@@ -142,8 +142,8 @@ def test_every_tile_bits(rt, tile, rows, cols, t):
 
 @pytest.mark.parametrize("kind,rows,cols,t,name", [
     ("product", 5232, 4352, 148, "gemm_tile<2, 2, 2, 1, 2, 2>"), ("product", 1024, 3072, 91, "gemm_mfma<"), ("product", 16, 8192, 200, "gemm_mfma<"),
-    ("norm", 5376, 3040, 116, "gemm_tile<4, 2, 2, 1, 2, 2>"), ("round_norm", 256, 1984, 60, "gemm_mfma_round<"), ("round_norm", 2480, 3072, 53, "gemm_mfma_round<"),
-    ("round_norm", 12288, 4096, 64, "gemm_tile<"), ("round", 8192, 4096, 65, "gemm_tile<"), ("round", 256, 4096, 65, "gemm_mfma_round<")])
+    ("norm", 5376, 3040, 116, "gemm_tile<"), ("round_norm", 256, 1984, 60, "gemm_mfma_round<"), ("round_norm", 2480, 3072, 53, "gemm_mfma_round<"),
+    ("round", 256, 4096, 65, "gemm_mfma_round<")])
 def test_the_rule(rt, kind, rows, cols, t, name):
     """Sizes at which another route was up to 1.9 times slower: tiles whose row tiles and token groups fill one
     XCD past its compute units, few rows (the 64-token launches split K over the device), and rounds of 65
@@ -248,26 +248,43 @@ def test_long_prompt_host_calls(rt, t):
         case.close()
 
 
-@pytest.mark.parametrize("rows,cols,t", [(12288, 4096, 64), (12288, 4096, 40), (6144, 1056, 33), (4096, 2048, 50)])
-def test_round_on_a_norm_up_to_64_tokens(rt, rows, cols, t):
-    """Rounds on a norm from 33 tokens: the norm in the limb image and the tiles, against the norm, the
-    64-token round and its sums apart, bit for bit (whichever the rule takes at these sizes)."""
-    case = Case(rt, rows, cols, t, rows + t)
+@pytest.mark.parametrize("shapes,cols,t,tile", [([8192, 4096, 32, 32], 4096, 64, True), ([8192, 4096, 32, 32], 4096, 33, False), ([4096, 4096, 4096, 48], 1056, 63, True),
+                                                ([12288, 16], 4096, 64, False), ([6144, 16], 1056, 33, False)])
+def test_round_on_a_norm_up_to_64_tokens(rt, shapes, cols, t, tile):
+    """Rounds on a norm from 33 tokens: the norm in the limb image and the tiles where that is the faster,
+    against the norm, the 64-token round and its sums apart, bit for bit. x rows apart."""
+    rng, n, xs = np.random.default_rng(t), len(shapes), cols + 12
+    q8 = [synth.q8_rows(rng, r, cols) for r in shapes]
+    x, nw = rng.standard_normal((t, xs)).astype(np.float32), (1.0 + 0.1 * rng.standard_normal(cols)).astype(np.float32)
+    w = [rt.upload(q, r, cols) for q, r in zip(q8, shapes)]
+    px, pn, py = rt.alloc(x.nbytes), rt.alloc(nw.nbytes), [rt.alloc(4 * t * r) for r in shapes]
+    rt.to_dev(px, x)
+    rt.to_dev(pn, nw)
+
+    def run():
+        rt.lib.rt_gemv_round_norm_dev(rt.R, n, (P * n)(*w), (c.c_long * n)(*shapes), cols, P(px), xs, t, P(pn), c.c_float(1e-6), (P * n)(*py))
+
+    def out():
+        got = [np.empty((t, r), np.float32) for r in shapes]
+        for a, p in zip(got, py):
+            rt.from_dev(a, p)
+        return got
+
     try:
-        case.nan()
-        name = kernels(rt, lambda: case.run("round_norm", 0, t))[0]
-        got = case.out()
+        name = kernels(rt, run)[0]
+        got = out()
         rt.set_epi_apart(True)
-        case.nan()
-        case.run("round_norm", 0, t)
-        rt.set_epi_apart(False)
-        print("round on a norm", rows, cols, t, name, flush=True)
-        assert rows != 12288 or t != 64 or name.startswith("gemm_tile<"), name
-        for a, b in zip(got, case.out()):
+        run()
+        print("round on a norm", shapes, cols, t, name, flush=True)
+        assert name.startswith("gemm_tile<" if tile else "gemm_mfma_"), name
+        for a, b in zip(got, out()):
             assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
     finally:
         rt.set_epi_apart(False)
-        case.close()
+        for p in (px, pn, *py):
+            rt.free(p)
+        for v in w:
+            rt.lib.rt_q8_free(rt.R, P(v))
 
 
 @pytest.mark.parametrize("t", [65, 68, 70])
