@@ -152,8 +152,9 @@ constexpr size_t KT_MAX = 16384;
 
 /* The workspace of a long prompt's limb image: 64 MiB hold 910 tokens of 12288 columns, 2730 of 4096;
  * longer prompts run in chunks of that many, each reading the weights again, which a chunk of
- * hundreds of tokens hides behind its arithmetic. Of one size, so that a graph may record any shape
- * once one long product has run. */
+ * hundreds of tokens hides behind its arithmetic. Of one size, so that a graph may record any shape on
+ * the tiles once one long product has run; the other routes record what 64 tokens' workspaces allow, 64
+ * tokens at a time. */
 constexpr long TILE_IMG_BYTES = 64L << 20;
 
 /* The runtimes alive, in the order rt_init set them up; rt_q8_row takes no struct rt
@@ -257,13 +258,19 @@ void reserve_staging(ctx *c, size_t nx, size_t ny)
     }
 }
 
-/* Workspace is allocated on demand, never while the stream is being recorded into a graph:
- * a product of a new, larger size must run once before a graph records it. */
-void no_capture(ctx *c, const char *what)
+bool recording(ctx *c)
 {
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     HIPCHECK(hipStreamIsCapturing(c->stream, &st));
-    if (st != hipStreamCaptureStatusNone)
+    return st != hipStreamCaptureStatusNone;
+}
+
+/* Workspace is allocated on demand, never while the stream is being recorded into a graph:
+ * a product of a new, larger size must run once before a graph records it (of more tokens than 64: at
+ * 64 or more). */
+void no_capture(ctx *c, const char *what)
+{
+    if (recording(c))
         failf(what, "must grow while a graph is being recorded: run a product of this size once before rt_graph_begin");
 }
 
@@ -320,13 +327,35 @@ float *reserve_round(ctx *c, int n, const long *rows, long cols, long t)
     return reserve_rpart(c, (size_t)q8_gemm_round_part_floats(n, rows, cols, t < 64 ? t : 64, c->gemm_opts));
 }
 
-/* the fused pair's two products (g) and their partials (rp) on the 64-token launches */
+/* the fused pair's two products (g), 64 tokens of them at a time, and their partials (rp) */
 void reserve_pair(ctx *c, long rows, long cols, long t, float **g, float **rp)
 {
     const long r2[2] = {rows, rows};
-    *g = reserve_scratch(c, (size_t)(2 * rows * t));
+    *g = reserve_scratch(c, (size_t)(2 * rows * (t < 64 ? t : 64)));
     *rp = reserve_round(c, 2, r2, cols, t);
 }
+
+/* The tiles need none of the 64-token launches' workspaces; an eager call leaves those of 64 tokens
+ * behind, as the launches would, for a later recording to count on */
+void tile_reserve(ctx *c, int n, const long *rows, long cols, long t, bool pair, bool norm)
+{
+    if (recording(c))
+        return;
+    float *g, *rp;
+    if (norm)
+        reserve_epi(c, (size_t)((t < 64 ? t : 64) * cols));
+    if (pair)
+        reserve_pair(c, rows[0], cols, t, &g, &rp);
+    else if (n > 1)
+        reserve_round(c, n, rows, cols, t);
+    else
+        reserve_gemm(c, rows[0], cols, 64);
+}
+
+/* Whether a recording has to take t tokens in parts, part i of n being [t i / n, t (i + 1) / n): more than
+ * 64 tokens for which the epilogue's workspace (width floats a token) is too small and must not grow. Parts
+ * of more than 64 tokens hold 33 or more, so that they stay on the matrix cores and keep their bits. */
+long record_parts(ctx *c, long t, long width) { return t > 64 && (size_t)(t * width) > c->epi_cap && recording(c) ? (t + 63) / 64 : 1; }
 
 /* Whether a product of t tokens runs on the matrix cores (every 64-token launch of it, the last
  * one too, however few tokens it holds, so that a token's bits do not depend on t), else on the
@@ -343,9 +372,7 @@ bool tile_ready(ctx *c, int n, const long *rows, long cols, long t, bool pair, b
         return false;
     if (part || c->ximg)
         return true;
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    HIPCHECK(hipStreamIsCapturing(c->stream, &st));
-    if (st != hipStreamCaptureStatusNone)
+    if (recording(c))
         return false;
     if (hipMalloc(&c->ximg, (size_t)TILE_IMG_BYTES) != hipSuccess) {
         (void)hipGetLastError();
@@ -385,7 +412,7 @@ void gemm_tokens(ctx *c, const void *w, long rows, long cols, const float *x, lo
     const q8_stream_t s = (q8_stream_t)c->stream;
     if (tile_ready(c, 1, &rows, cols, t, false, false, part)) {
         if (!part)
-            reserve_gemm(c, rows, cols, 64); /* as the 64-token launches: a later recording may count on it */
+            tile_reserve(c, 1, &rows, cols, t, false, false);
         tile_run(c, 1, &w, &rows, cols, x, xs, t, &y, res, nullptr, nullptr, 0.0f, part);
         return;
     }
@@ -427,10 +454,13 @@ void product(ctx *c, const void *w0, const void *w1, long rows, long cols, const
         if (!w1) {
             q8_launch_exact(s, w0, rows, cols, x, xs, t, y);
         } else {
-            float *g = reserve_scratch(c, (size_t)(2 * rows * t));
-            q8_launch_exact(s, w0, rows, cols, x, xs, t, g);
-            q8_launch_exact(s, w1, rows, cols, x, xs, t, g + rows * t);
-            q8_launch_swiglu_ew(s, g, g + rows * t, rows * t, y);
+            float *g = reserve_scratch(c, (size_t)(2 * rows * (t < 64 ? t : 64)));
+            for (long k = 0; k < t; k += 64) {
+                const long n = t - k < 64 ? t - k : 64;
+                q8_launch_exact(s, w0, rows, cols, x + k * xs, xs, n, g);
+                q8_launch_exact(s, w1, rows, cols, x + k * xs, xs, n, g + rows * n);
+                q8_launch_swiglu_ew(s, g, g + rows * n, rows * n, y + k * rows);
+            }
         }
         launched("the reference-order product");
         return;
@@ -440,18 +470,19 @@ void product(ctx *c, const void *w0, const void *w1, long rows, long cols, const
     } else if (!w1) {
         gemm_tokens(c, w0, rows, cols, x, xs, t, y, nullptr, part);
     } else {
-        float *g, *rp;
-        reserve_pair(c, rows, cols, t, &g, &rp);
         /* 64 tokens at a time, the gate and the up product as one round, their sums and the SwiGLU
          * in one launch: the same sums and SwiGLU as apart (below, where the round is refused) */
         const void *w2[2] = {w0, w1};
         const long r2[2] = {rows, rows};
         bool pair_done = true;
         if (tile_ready(c, 2, r2, cols, t, true, false, nullptr)) {
+            tile_reserve(c, 2, r2, cols, t, true, false);
             tile_run(c, 2, w2, r2, cols, x, xs, t, nullptr, nullptr, y, nullptr, 0.0f, nullptr);
             launched("the fused pair");
             return;
         }
+        float *g, *rp;
+        reserve_pair(c, rows, cols, t, &g, &rp);
         for (long k = 0; k < t && pair_done; k += 64) {
             const long tk = t - k < 64 ? t - k : 64;
             float *y2[2] = {g, g + rows * tk};
@@ -465,9 +496,12 @@ void product(ctx *c, const void *w0, const void *w1, long rows, long cols, const
             launched("the fused pair");
             return;
         }
-        gemm_tokens(c, w0, rows, cols, x, xs, t, g);
-        gemm_tokens(c, w1, rows, cols, x, xs, t, g + rows * t);
-        q8_launch_swiglu_ew(s, g, g + rows * t, rows * t, y);
+        for (long k = 0; k < t; k += 64) {
+            const long n = t - k < 64 ? t - k : 64;
+            gemm_tokens(c, w0, rows, cols, x + k * xs, xs, n, g);
+            gemm_tokens(c, w1, rows, cols, x + k * xs, xs, n, g + rows * n);
+            q8_launch_swiglu_ew(s, g, g + rows * n, rows * n, y + k * rows);
+        }
     }
     launched("the product");
 }
@@ -503,7 +537,7 @@ bool overlaps(const float *x, long xs, long t, long cols, const float *y, long n
 void product_epi(ctx *c, const void *w0, const void *w1, long rows, long cols, const float *x, long xs, long t, float *y, q8_epi e)
 {
     const q8_stream_t s = (q8_stream_t)c->stream;
-    const bool apart = c->epi_apart != 0 || ((e.nw || t <= 4) && overlaps(x, xs, t, cols, y, t * rows));
+    const bool over = overlaps(x, xs, t, cols, y, t * rows), apart = c->epi_apart != 0 || ((e.nw || t <= 4) && over);
     if (!c->exact && t <= 4 && !apart) {
         const bool timed = kt_begin(c, RT_K_GEMV + (w1 ? 1 : 0), rows, cols, t);
         if (q8_launch_gemv_epi(s, w0, w1, rows, cols, x, xs, t, y, e) == 0) {
@@ -514,23 +548,23 @@ void product_epi(ctx *c, const void *w0, const void *w1, long rows, long cols, c
             kt_cancel(c);
     }
     if (e.nw) {
-        float *xn = reserve_epi(c, (size_t)(t * cols));
         const void *w2[2] = {w0, w1};
         const long r2[2] = {rows, rows};
         if (!c->exact && !apart && tile_ready(c, w1 ? 2 : 1, r2, cols, t, w1 != nullptr, true, nullptr)) {
-            /* the norm in the limb image: the same sum and the same xn as apart. The workspaces as
-             * product() reserves them: a later recording of fewer tokens may count on them */
-            if (w1) {
-                float *g, *rp;
-                reserve_pair(c, rows, cols, t, &g, &rp);
-            } else {
-                reserve_gemm(c, rows, cols, 64);
-            }
+            /* the norm in the limb image: the same sum and the same xn as apart */
+            tile_reserve(c, w1 ? 2 : 1, r2, cols, t, w1 != nullptr, true);
             kt_begin(c, w1 ? RT_K_GEMM_PAIR : RT_K_GEMM, rows, cols, t);
             tile_run(c, w1 ? 2 : 1, w2, r2, cols, x, xs, t, &y, nullptr, w1 ? y : nullptr, e.nw, e.eps, nullptr);
             launched("the product on the norm");
             return;
         }
+        const long parts = over ? 1 : record_parts(c, t, cols);
+        if (parts > 1) {
+            for (long i = 0; i < parts; i++)
+                product_epi(c, w0, w1, rows, cols, x + t * i / parts * xs, xs, t * (i + 1) / parts - t * i / parts, y + t * i / parts * rows, e);
+            return;
+        }
+        float *xn = reserve_epi(c, (size_t)(t * cols));
         q8_launch_rmsnorm(s, x, xs, t, cols, e.nw, e.eps, xn);
         launched("the norm");
         product(c, w0, w1, rows, cols, xn, cols, t, y);
@@ -540,6 +574,14 @@ void product_epi(ctx *c, const void *w0, const void *w1, long rows, long cols, c
         kt_begin(c, RT_K_GEMM, rows, cols, t);
         gemm_tokens(c, w0, rows, cols, x, xs, t, y, e.res);
         launched("the product and its residual");
+        return;
+    }
+    const long parts = over ? 1 : record_parts(c, t, rows);
+    if (parts > 1) {
+        for (long i = 0; i < parts; i++) {
+            const long k = t * i / parts;
+            product_epi(c, w0, w1, rows, cols, x + k * xs, xs, t * (i + 1) / parts - k, y + k * rows, q8_epi{nullptr, 0.0f, e.res + k * rows});
+        }
         return;
     }
     float *tmp = reserve_epi(c, (size_t)(t * rows));
@@ -569,13 +611,14 @@ bool round_launch(ctx *c, int n, const void *const *w, const long *rows, long co
         rc = q8_launch_gemv_round((q8_stream_t)c->stream, n, w, rows, cols, x, xs, t, y);
     } else {
         /* 64 tokens at a time (a token's bits do not depend on t) */
-        float *rp = reserve_round(c, n, rows, cols, t);
         rc = 0;
         if (tile_ready(c, n, rows, cols, t, false, false, nullptr)) {
+            tile_reserve(c, n, rows, cols, t, false, false);
             tile_run(c, n, w, rows, cols, x, xs, t, y, nullptr, nullptr, nullptr, 0.0f, nullptr);
             launched("the round");
             return true;
         }
+        float *rp = reserve_round(c, n, rows, cols, t);
         for (long k = 0; k < t && rc == 0; k += 64) {
             const long tk = t - k < 64 ? t - k : 64;
             float *yk[RT_BATCH];
@@ -1164,9 +1207,10 @@ void rt_gemv_round_norm_dev(struct rt *R, int n, const void *const *w, const lon
         check_dev_ptr("rt_gemv_round_norm_dev", y[i], "every y");
     }
     const q8_stream_t s = (q8_stream_t)c->stream;
-    bool apart = c->epi_apart != 0;
+    bool over = false;
     for (int i = 0; i < n; i++)
-        apart = apart || overlaps(x, x_stride, t, cols, y[i], t * rows[i]);
+        over = over || overlaps(x, x_stride, t, cols, y[i], t * rows[i]);
+    const bool apart = c->epi_apart != 0 || over;
     if (!c->exact && t <= 4 && !apart) {
         long total = 0;
         for (int i = 0; i < n; i++)
@@ -1179,9 +1223,8 @@ void rt_gemv_round_norm_dev(struct rt *R, int n, const void *const *w, const lon
         if (timed)
             kt_cancel(c);
     }
-    float *xn = reserve_epi(c, (size_t)(t * cols));
     if (!c->exact && n > 1 && !apart && tile_ready(c, n, rows, cols, t, false, true, nullptr)) {
-        reserve_round(c, n, rows, cols, t);
+        tile_reserve(c, n, rows, cols, t, false, true);
         long total = 0;
         for (int i = 0; i < n; i++)
             total += rows[i];
@@ -1190,6 +1233,18 @@ void rt_gemv_round_norm_dev(struct rt *R, int n, const void *const *w, const lon
         launched("the round on the norm");
         return;
     }
+    const long parts = over ? 1 : record_parts(c, t, cols);
+    if (parts > 1) {
+        for (long i = 0; i < parts; i++) {
+            const long k = t * i / parts;
+            float *yk[RT_BATCH];
+            for (int j = 0; j < n; j++)
+                yk[j] = y[j] + k * rows[j];
+            rt_gemv_round_norm_dev(R, n, w, rows, cols, x + k * x_stride, x_stride, t * (i + 1) / parts - k, nw, eps, yk);
+        }
+        return;
+    }
+    float *xn = reserve_epi(c, (size_t)(t * cols));
     q8_launch_rmsnorm(s, x, x_stride, t, cols, nw, eps, xn);
     launched("the norm");
     if (!c->exact && n > 1 && round_launch(c, n, w, rows, cols, xn, cols, t, y))

@@ -349,3 +349,39 @@ def test_round_sums_of_many_outputs(rt, cols):
             rt.free(p)
         for v in w:
             rt.lib.rt_q8_free(rt.R, P(v))
+
+
+@pytest.mark.parametrize("rows,cols,first,t", [(1024, 1024, 66, 500), (64, 2048, 64, 210), (64, 2048, 70, 130), (2048, 1056, 130, 131)])
+@pytest.mark.parametrize("exact", [False, True])
+def test_recorded_at_more_tokens_than_ran(q8rt, rt, rows, cols, first, t, exact):
+    """A runtime that ran each product once, at 64 tokens or a few more, records them at more: on the tiles,
+    which need no workspace but the image, or 64 tokens at a time where the rule refuses them (64 rows).
+    Replayed twice with eager work between, bit for bit the eager products."""
+    kinds = ("product", "residual", "norm", "pair", "pair_norm", "round", "round_norm")
+    want, case = {}, Case(rt, rows, cols, t, 31)
+    rt.set_exact(exact)
+    try:
+        for kind in kinds:
+            case.nan()
+            case.run(kind, 0, t)
+            want[kind] = case.out()
+    finally:
+        rt.set_exact(False)
+        case.close()
+    with q8rt.Runtime() as r2:
+        r2.set_exact(exact)
+        c2 = Case(r2, rows, cols, t, 31)
+        for kind in kinds:
+            c2.run(kind, 0, first)
+        for kind in kinds:
+            r2.lib.rt_graph_begin(r2.R)
+            c2.run(kind, 0, t)
+            g = P(r2.lib.rt_graph_end(r2.R))
+            for _ in range(2):
+                c2.run("pair", 0, 5)
+                c2.nan()
+                r2.lib.rt_graph_launch(r2.R, g)
+                for a, b in zip(c2.out(), want[kind]):
+                    assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), kind
+            r2.lib.rt_graph_free(r2.R, g)
+        c2.close()
