@@ -720,17 +720,46 @@ void run_round(ctx *c, job *jobs, int n, const char *what)
     bool direct = c->x_direct && !c->exact;
     for (int i = 0; i < n; i++)
         direct = direct && jobs[i].t <= 4;
-    /* Long prompts store y into HBM and a copy kernel moves it, a KiB a wave: the tiles' own stores are 64
-     * bytes of a token's row each, and over the host link they took 1077 us at 512 tokens of 12288 x
-     * 4096 against 868 for the 64-token launches' sums and 809 through the copy. */
+    /* products that share x (and t): one round for the group */
+    struct {
+        int n, idx[RT_BATCH];
+        long rows[RT_BATCH];
+    } group[RT_BATCH];
+    int groups = 0;
+    bool grouped[RT_BATCH] = {};
+    for (int i = 0; i < n; i++) {
+        if (grouped[i])
+            continue;
+        auto &g = group[groups++];
+        g.n = 0;
+        for (int j = i; j < n; j++)
+            if (j == i || (!c->exact && !grouped[j] && jobs[j].x_off == jobs[i].x_off && jobs[j].t == jobs[i].t && jobs[j].cols == jobs[i].cols)) {
+                grouped[j] = true;
+                g.idx[g.n] = j, g.rows[g.n++] = jobs[j].rows;
+            }
+    }
+    /* What the tiles compute (long prompts) goes into HBM and a copy kernel moves it, a KiB a wave: the tiles'
+     * own stores are 64 bytes of a token's row each, and over the host link they took 1077 us at 512 tokens
+     * of 12288 x 4096 against 868 for the 64-token launches' sums and 809 through the copy. The sums' own
+     * stores stay: 256 x 4096 at 200 tokens 184 us, 198 through the copy. */
     bool far = false;
-    for (int i = 0; i < n; i++)
-        far = far || (jobs[i].t > 64 && !c->exact);
+    for (int k = 0; k < groups; k++) {
+        const job &j = jobs[group[k].idx[0]];
+        far = far || (!c->exact && q8_tile_takes(group[k].n, group[k].rows, j.cols, j.t, false, false, c->gemm_opts));
+    }
     if (far && ny > c->dy_cap) {
         if (c->dy)
             HIPCHECK(hipFree(c->dy));
-        c->dy_cap = ny + ny / 2;
-        HIPCHECK(hipMalloc((void **)&c->dy, c->dy_cap * sizeof(float)));
+        c->dy = nullptr;
+        c->dy_cap = 0;
+        /* without room for it y goes over the link from the kernels */
+        if (hipMalloc((void **)&c->dy, (ny + ny / 2) * sizeof(float)) == hipSuccess) {
+            c->dy_cap = ny + ny / 2;
+        } else {
+            (void)hipGetLastError();
+            c->dy = nullptr;
+            far = false;
+        }
     }
     float *yb = far ? c->dy : c->hy;
     const float *xb = c->dx;
@@ -740,27 +769,17 @@ void run_round(ctx *c, job *jobs, int n, const char *what)
         q8_launch_copy((q8_stream_t)c->stream, c->dx, c->hx, (long)(nx / 4)); /* nx is a multiple of 64 floats */
         launched("the copy of x");
     }
-    /* products that share x (and t): one round for the group */
-    bool done[RT_BATCH] = {};
-    for (int i = 0; i < n && !c->exact; i++) {
-        if (done[i])
-            continue;
+    for (int k = 0; k < groups; k++) {
+        const auto &g = group[k];
+        const job &j0 = jobs[g.idx[0]];
         const void *w[RT_BATCH];
-        long rows[RT_BATCH];
         float *y[RT_BATCH];
-        int idx[RT_BATCH], k = 0;
-        for (int j = i; j < n; j++)
-            if (!done[j] && jobs[j].x_off == jobs[i].x_off && jobs[j].t == jobs[i].t && jobs[j].cols == jobs[i].cols) {
-                w[k] = jobs[j].w, rows[k] = jobs[j].rows, y[k] = yb + jobs[j].y_off, idx[k++] = j;
-            }
-        if (k > 1 && round_launch(c, k, w, rows, jobs[i].cols, xb + jobs[i].x_off, jobs[i].cols, jobs[i].t, y))
-            for (int j = 0; j < k; j++)
-                done[idx[j]] = true;
-    }
-    for (int i = 0; i < n; i++) {
-        const job &j = jobs[i];
-        if (!done[i])
-            product(c, j.w, nullptr, j.rows, j.cols, xb + j.x_off, j.cols, j.t, yb + j.y_off);
+        for (int i = 0; i < g.n; i++)
+            w[i] = jobs[g.idx[i]].w, y[i] = yb + jobs[g.idx[i]].y_off;
+        if (g.n > 1 && round_launch(c, g.n, w, g.rows, j0.cols, xb + j0.x_off, j0.cols, j0.t, y))
+            continue;
+        for (int i = 0; i < g.n; i++)
+            product(c, w[i], nullptr, g.rows[i], j0.cols, xb + j0.x_off, j0.cols, j0.t, y[i]);
     }
     if (far) {
         q8_launch_copy((q8_stream_t)c->stream, c->hy, c->dy, (long)(ny / 4)); /* ny is a multiple of 64 floats */

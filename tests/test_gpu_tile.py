@@ -225,24 +225,25 @@ def test_long_prompt_recorded(q8rt, rt):
         c2.close()
 
 
+@pytest.mark.parametrize("rows,cols", [(1040, 1056), (64, 2048)])
 @pytest.mark.parametrize("t", [65, 130, 300])
-def test_long_prompt_host_calls(rt, t):
-    """rt_gemm, and two products queued with another of one token, on host arrays: y goes through HBM at
-    more than 64 tokens; bit for bit the device products, with x and y sizes that grow and shrink."""
-    case = Case(rt, 1040, 1056, t, 21 + t)
+def test_long_prompt_host_calls(rt, t, rows, cols):
+    """rt_gemm, and two products queued with another of one token, on host arrays: y goes through HBM
+    where the tiles run and over the link from the sums where they do not (64 rows); bit for bit the device products, with x and y sizes that grow and shrink."""
+    case = Case(rt, rows, cols, t, 21 + t)
     try:
         case.run("product", 0, t)
         want = case.out()[0]
-        y = [np.full((t, 1040), np.nan, np.float32) for _ in range(3)]
-        x1, y1 = np.ascontiguousarray(case.x[:1]), np.full((1, 1040), np.nan, np.float32)
-        rt.gemm(case.w[0], 1040, 1056, case.x, t, y[0])
-        rt.gemm_q(case.w[0], 1040, 1056, case.x, t, y[1])
-        rt.gemv_q(case.w[1], 1040, 1056, x1, y1)
-        rt.gemm_q(case.w[0], 1040, 1056, case.x, t, y[2])
+        y = [np.full((t, rows), np.nan, np.float32) for _ in range(3)]
+        x1, y1 = np.ascontiguousarray(case.x[:1]), np.full((1, rows), np.nan, np.float32)
+        rt.gemm(case.w[0], rows, cols, case.x, t, y[0])
+        rt.gemm_q(case.w[0], rows, cols, case.x, t, y[1])
+        rt.gemv_q(case.w[1], rows, cols, x1, y1)
+        rt.gemm_q(case.w[0], rows, cols, case.x, t, y[2])
         rt.gemv_go()
         for a in y:
             assert np.array_equal(a.view(np.uint32), want.view(np.uint32))
-        rt.lib.rt_gemv_dev(rt.R, P(case.w[1]), 1040, 1056, P(case.p["x"]), P(case.y))
+        rt.lib.rt_gemv_dev(rt.R, P(case.w[1]), rows, cols, P(case.p["x"]), P(case.y))
         assert np.array_equal(case.out()[0][0].view(np.uint32), y1[0].view(np.uint32))
     finally:
         case.close()
