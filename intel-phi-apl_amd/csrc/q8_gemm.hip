@@ -712,10 +712,11 @@ __global__ __launch_bounds__(64 * NW) void read_xres(const uint8_t *w, long rows
 /* The sum of an output's ks partials (splits step floats apart), in split order: sixteen splits' loads
  * in flight at a time, all issued before the first add (past the last split the index is clamped and
  * the value not added). V: an output a thread (float), or four neighbouring ones (float4; rows are
- * whole 16s) where that still gives every compute unit three workgroups, sum_vec: at 64 tokens the round
+ * whole 16s) where that still gives every compute unit three workgroups, or two with few units
+ * short of one, sum_vec: at 64 tokens the round
  * of 12320 rows (33 MB of partials) 9.3 us against 9.9 with one, the 12288-row pair 7.1 against 8.3, the
- * product 16384 x 4096 with its sums 42.0 against 43.5. On fewer outputs, a last workgroup on some units
- * alone, and where a product has more than 32 splits (few rows of many columns, each thread's chain of
+ * product 16384 x 4096 with its sums 42.0 against 43.5, 8192 x 4096 27.8 against 28.8. On fewer outputs, a
+ * last workgroup on some units alone (the pair 9216 x 4096 60.4 against 59.3), and where a product has more than 32 splits (few rows of many columns, each thread's chain of
  * adds four times as wide), one a thread is the faster: the round 4096 + 32 + 32 rows of 10240 columns at
  * 64 tokens 42.4 us against 46.3, 12288 + 32 + 32 87.3 against 89.8. */
 __device__ __forceinline__ float4 sum_add(float4 a, float4 b) { return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w); }
@@ -742,7 +743,11 @@ __device__ __forceinline__ V split_sum(const float *__restrict__ part, int ks, l
     return v;
 }
 /* the outputs a thread of a sum of n outputs, and its grid */
-static bool sum_vec(long n, int ks) { return n >= 3L * 4 * 256 * 256 && ks <= 32; }
+static bool sum_vec(long n, int ks)
+{
+    const long unit = 4L * 256 * 256, most = (n + unit - 1) / unit; /* the outputs of a workgroup a unit; a unit's workgroups */
+    return ks <= 32 && (n >= 3 * unit || (most == 2 && 10 * most * unit <= 11 * n));
+}
 static dim3 sum_grid(long n, bool vec) { return dim3((unsigned)(((vec ? n / 4 : n) + 255) / 256)); }
 template <class V>
 __device__ __forceinline__ long sum_first()
