@@ -1,7 +1,7 @@
 """Products of more than 64 tokens as one launch (csrc/q8_tile.hip) against the 64-token launches,
-bit for bit: the same sums in the same order, at every tile configuration, partial tiles of rows and
-tokens, odd block counts (half a last pair, 2-byte aligned scales), forced K splits (one, and a
-shorter last one), the residual, the norm, the fused pair, rounds, non-finite x and scales, chunks of
+bit for bit: the same sums in the same order, at every tile configuration (by name), partial tiles of rows and
+tokens, x rows apart, odd block counts (half a last pair, 2-byte aligned scales), forced K splits (one, and a
+shorter last one), the residual (in place too), the norm, the fused pair, rounds, non-finite x and scales, chunks of
 the limb image, and under graph capture."""
 import ctypes as c
 
@@ -29,9 +29,10 @@ def kernels(rt, fn):
 
 
 class Case:
-    """Two matrices and x on the device; run(kind, k, n) is one call on tokens [k, k + n)."""
+    """Two matrices and x on the device (its rows cols + pad floats apart); run(kind, k, n) is one call on
+    tokens [k, k + n)."""
 
-    def __init__(self, rt, rows, cols, t, seed, x=None, q8=None):
+    def __init__(self, rt, rows, cols, t, seed, x=None, q8=None, pad=0):
         rng = np.random.default_rng(seed)
         self.rt, self.rows, self.cols, self.t = rt, rows, cols, t
         self.q8 = q8 or [synth.q8_rows(rng, rows, cols) for _ in range(2)]
@@ -39,7 +40,8 @@ class Case:
         self.nw = (1.0 + 0.1 * rng.standard_normal(cols)).astype(np.float32)
         self.res = rng.standard_normal((t, rows)).astype(np.float32)
         self.w = [rt.upload(q, rows, cols) for q in self.q8]
-        self.p = {k: self.put(v) for k, v in (("x", self.x), ("nw", self.nw), ("res", self.res))}
+        self.xs = cols + pad
+        self.p = {k: self.put(v) for k, v in (("x", np.pad(self.x, ((0, 0), (0, pad)), constant_values=np.nan)), ("nw", self.nw), ("res", self.res))}
         self.y, self.z = rt.alloc(4 * t * rows), rt.alloc(4 * t * 16)
 
     def put(self, a):
@@ -55,27 +57,30 @@ class Case:
 
     def run(self, kind, k, n):
         lib, R, rows, cols, eps = self.rt.lib, self.rt.R, self.rows, self.cols, c.c_float(1e-6)
-        x, y, nw, res = P(self.p["x"] + 4 * k * cols), P(self.y + 4 * k * rows), P(self.p["nw"]), P(self.p["res"] + 4 * k * rows)
+        xs = self.xs
+        x, y, nw, res = P(self.p["x"] + 4 * k * xs), P(self.y + 4 * k * rows), P(self.p["nw"]), P(self.p["res"] + 4 * k * rows)
         w = [P(v) for v in self.w]
         if kind == "product":
-            lib.rt_gemm_dev(R, w[0], rows, cols, x, cols, n, y)
+            lib.rt_gemm_dev(R, w[0], rows, cols, x, xs, n, y)
         elif kind == "noalloc":
-            lib.rt_gemm_dev_noalloc(R, w[0], rows, cols, x, cols, n, y)
+            lib.rt_gemm_dev_noalloc(R, w[0], rows, cols, x, xs, n, y)
         elif kind == "residual":
-            lib.rt_gemm_residual_dev(R, w[0], rows, cols, x, cols, n, res, y)
+            lib.rt_gemm_residual_dev(R, w[0], rows, cols, x, xs, n, res, y)
+        elif kind == "inplace":  # the residual in y itself
+            lib.rt_gemm_residual_dev(R, w[0], rows, cols, x, xs, n, y, y)
         elif kind == "norm":
-            lib.rt_gemm_norm_dev(R, w[0], rows, cols, x, cols, n, nw, eps, y)
+            lib.rt_gemm_norm_dev(R, w[0], rows, cols, x, xs, n, nw, eps, y)
         elif kind == "pair":
-            lib.rt_gemv_swiglu_dev(R, w[0], w[1], rows, cols, x, cols, n, y)
+            lib.rt_gemv_swiglu_dev(R, w[0], w[1], rows, cols, x, xs, n, y)
         elif kind == "pair_norm":
-            lib.rt_gemv_swiglu_norm_dev(R, w[0], w[1], rows, cols, x, cols, n, nw, eps, y)
+            lib.rt_gemv_swiglu_norm_dev(R, w[0], w[1], rows, cols, x, xs, n, nw, eps, y)
         else:  # rounds: the matrix and a 16-row prefix of the other
             ws, rr = (P * 2)(self.w[0], self.w[1]), (c.c_long * 2)(rows, 16)
             ys = (P * 2)(self.y + 4 * k * rows, self.z + 4 * k * 16)
             if kind == "round":
-                lib.rt_gemv_round_dev(R, 2, ws, rr, cols, x, cols, n, ys)
+                lib.rt_gemv_round_dev(R, 2, ws, rr, cols, x, xs, n, ys)
             else:
-                lib.rt_gemv_round_norm_dev(R, 2, ws, rr, cols, x, cols, n, nw, eps, ys)
+                lib.rt_gemv_round_norm_dev(R, 2, ws, rr, cols, x, xs, n, nw, eps, ys)
 
     def out(self):
         y, z = np.empty((self.t, self.rows), np.float32), np.empty((self.t, 16), np.float32)
@@ -88,18 +93,22 @@ class Case:
         self.rt.to_dev(self.z, np.full((self.t, 16), np.nan, np.float32))
 
     def whole_and_parts(self, kind):
-        """(kernel name, outputs of one call, outputs of 64-token calls; a last call holds 5 tokens or more)"""
+        """(kernel name, outputs of one call, outputs of calls of up to 64 tokens and 5 or more)"""
         self.nan()
+        if kind == "inplace":
+            self.rt.to_dev(self.y, self.res)
         names = kernels(self.rt, lambda: self.run(kind, 0, self.t))
         one = self.out()
         self.nan()
-        for k in range(0, self.t, 64):
-            k = min(k, max(0, self.t - 5))
-            self.run(kind, k, min(64, self.t - k))
+        if kind == "inplace":
+            self.rt.to_dev(self.y, self.res)
+        step = 64 if self.t % 64 == 0 or self.t % 64 >= 5 else 59  # every call on the matrix cores, no token twice
+        for k in range(0, self.t, step):
+            self.run(kind, k, min(step, self.t - k))
         return names[0], one, self.out()
 
 
-KINDS = ("product", "noalloc", "residual", "norm", "pair", "pair_norm", "round", "round_norm")
+KINDS = ("product", "noalloc", "residual", "inplace", "norm", "pair", "pair_norm", "round", "round_norm")
 # (rows, cols, tokens, forced K splits): the tiles' edges. 512 x 4096 rows fill the device with the
 # small tiles and 12288 with the large ones
 SHAPES = [(256, 64, 300, 0), (512, 96, 2000, 0), (1888, 1056, 131, 0), (1888, 1056, 500, 3), (1888, 1056, 200, 1), (2048, 6144, 203, 0), (2048, 2048, 203, 5), (4096, 1024, 513, 1), (5136, 2784, 300, 0),
@@ -108,7 +117,7 @@ SHAPES = [(256, 64, 300, 0), (512, 96, 2000, 0), (1888, 1056, 131, 0), (1888, 10
 
 @pytest.mark.parametrize("rows,cols,t,ks", SHAPES)
 def test_long_prompt_bits(rt, rows, cols, t, ks):
-    case = Case(rt, rows, cols, t, rows + cols + t)
+    case = Case(rt, rows, cols, t, rows + cols + t, pad=4 * (rows % 7))
     rt.gemm_force(False, ks)
     try:
         for kind in KINDS:
