@@ -142,8 +142,8 @@ void rt_gemm_dev(struct rt *R, const void *w, long rows, long cols, const float 
 /* rt_gemm_dev that allocates nothing, for callers that cannot call hipMalloc (code under HIP graph
  * capture, tight serving loops, harnesses that forbid allocation). No counterpart in the reference.
  * The same kernels and the same results, bit for bit; the matrix-core product's K-split partials
- * (t >= 5) live in a static device array of the library, 32 MiB (8 Mi floats) on every GPU it runs
- * on, held until the process ends. A product whose partials would exceed it is refused with the
+ * (t >= 5), or a long prompt's x as the tiles read it, live in a static device array of the library,
+ * 32 MiB (8 Mi floats) on every GPU it runs on, held until the process ends. A product whose partials would exceed it is refused with the
  * reason. Every call on a GPU shares that GPU's array: calls that overlap on one GPU (two streams,
  * two runtimes) race. */
 void rt_gemm_dev_noalloc(struct rt *R, const void *w, long rows, long cols, const float *x, long x_stride, long t, float *y);
@@ -158,14 +158,16 @@ void rt_gemv_round_dev(struct rt *R, int n, const void *const *w, const long *ro
 /* The FFN's fused pair: Y[k] = SiLU(G[k]) * U[k] with G = X Wg^T and U = X Wu^T, both [rows cols],
  * x read once for both; SiLU(g) = g / (1 + exp(-g)) (src/apl/qwen35.apl:38, 125). t tokens: up to
  * 4 one decode launch; from 5, 64 tokens at a time, the two products as a matrix-core round and
- * their sums with the SwiGLU in one more launch. */
+ * their sums with the SwiGLU in one more launch, or one launch for all of a long prompt (more than 64
+ * tokens, where that is the faster). */
 void rt_gemv_swiglu_dev(struct rt *R, const void *wg, const void *wu, long rows, long cols, const float *x, long x_stride, long t, float *y);
 /* ---- the epilogues on either side of a product (additions; the reference computes them on its
  * host around the products: RMS = {⍺×⍵×(RMS_EPS+(+/⍵×⍵)÷≢⍵)*¯0.5}, src/apl/qwen35.apl:49, before a
  * layer's mixer and FFN, and the residual Z←X+… after them, qwen35.apl:131-139). Fused into the
- * decode kernel (t <= 4; the norm up to 8192 columns and at 12288, the residual up to 16384), the residual
- * into the matrix-core product's for t >= 5 and the norm into a long prompt's (more than 64 tokens);
- * otherwise the norm or the add runs as a kernel of its own. The
+ * decode kernel (t <= 4; the norm up to 8192 columns and at 12288, the residual up to 16384, but on many
+ * rows of more than 4096 columns at 2 to 4 tokens, where apart is the faster), the residual into the
+ * matrix-core product's for t >= 5 and the norm into a long prompt's one launch (more than 64 tokens;
+ * rounds on a norm more than 32); otherwise the norm or the add runs as a kernel of its own. The
  * norm is s = 1 / sqrt(eps + sum_k x[k]^2 / cols) per token in F32, xn[k] = nw[k] * (x[k] * s); its
  * sum runs in a fixed order for a given shape, so results repeat bit for bit, and a fused and a
  * separate norm differ only by that order (an ulp or so of s). The residual is one F32 add of the
@@ -180,7 +182,8 @@ void rt_gemm_norm_dev(struct rt *R, const void *w, long rows, long cols, const f
 void rt_gemv_swiglu_norm_dev(struct rt *R, const void *wg, const void *wu, long rows, long cols, const float *x, long x_stride, long t, const float *nw,
                              float eps, float *y);
 /* A round of products sharing RMS(X) (the DeltaNet quartet on W_ANORM RMS X): at t <= 4 one
- * launch with the norm fused; from 5 tokens the norm, then the round's launches as above. */
+ * launch with the norm fused; from 5 tokens the norm, then the round's launches as above, or from 33 both
+ * as one, where that is the faster. */
 void rt_gemv_round_norm_dev(struct rt *R, int n, const void *const *w, const long *rows, long cols, const float *x, long x_stride, long t,
                             const float *nw, float eps, float *const *y);
 /* Y = R + X W^T (after W_OUT and W_DOWN); r [t rows] may be y, the residual stream updated in place. */
@@ -205,7 +208,8 @@ void rt_dev_sync(struct rt *R);
 /* A recorded sequence of device products, replayed with one call (a HIP graph captured from
  * the runtime's stream): rt_graph_begin, then any rt_*_dev products (no host-pointer products,
  * no copies), then rt_graph_end returns the sequence; rt_graph_launch enqueues one replay on the
- * stream, in order with every other product. The pointers recorded are used as they are. */
+ * stream, in order with every other product. The pointers recorded are used as they are. Workspaces do not
+ * grow while recording: run each product once before, at as many tokens or at 64 or more. */
 void rt_graph_begin(struct rt *R);
 void *rt_graph_end(struct rt *R);
 void rt_graph_launch(struct rt *R, void *graph);

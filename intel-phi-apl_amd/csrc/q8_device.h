@@ -249,7 +249,8 @@ bool q8_launch_round_any(q8_stream_t stream, const q8_round &r, long cols, const
 void q8_launch_rmsnorm(q8_stream_t stream, const float *x, long x_stride, long t, long cols, const float *nw, float eps, float *xn);
 /* y[i] = a[i] + b[i], i < n (y may be a or b). */
 void q8_launch_add(q8_stream_t stream, const float *a, const float *b, long n, float *y);
-/* A round of products sharing x as one launch (t <= 4, cols % 1024 == 0, every rows % 8 == 0):
+/* A round of products sharing x as one launch (t <= 4, cols up to 16384, at 3 and 4 tokens up to 12288 and
+ * where gemv_round has an instance; every rows % 8 == 0):
  * 0, or -1 (nothing launched: the caller runs them one by one). */
 #define Q8_ROUND_MAX 8
 #define Q8_ROUND_RW 8 /* rows a workgroup of a decode round */

@@ -1,11 +1,11 @@
 /* q8_gemv_any.hip: the decode kernels (t = 1..4) for any cols, a multiple of 32 up to 16384: matrices
  * whose K is no multiple of 1024, and the epilogues at the multiples that q8_kernels.hip has no fused
- * instance for. The body is the same (q8_gemv.h) on ceil(cols / 1024) waves a workgroup; the last
- * wave's lanes past the row count as zero.
+ * instance for. The body is the same (q8_gemv.h) on one wave a started 1024 columns, the last wave's lanes
+ * past the row counting as zero, or on 4, 8 or 12 whole ones and a tail (q8_any_waves).
  *
  * HBM-bound like the others: every load of a workgroup's rows is issued before any arithmetic, where
  * the loop over K (gemv_s, for more than 16384 columns now) keeps 4 rows' loads of one 1024-column
- * step in flight. The pair 11008 x 4128 at 3
+ * step in flight. The pair 11008 x 4128 (4 waves and a tail) at 3
  * tokens 35.1 -> 25.2 us (3.84 TB/s of weights); one-token pair 5424 x 4256 16.9 -> 10.5; a layer of
  * 1536 columns with its epilogues, which ran apart at such sizes, at 2 tokens 41.8 -> 17.4 us. With
  * a fifth wave for the two units that 4128 columns have past 4096 the pair took 39.7 us, slower than

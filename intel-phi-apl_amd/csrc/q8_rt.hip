@@ -363,8 +363,7 @@ long record_parts(ctx *c, long t, long width) { return t > 64 && (size_t)(t * wi
 bool on_matrix_cores(long t) { return t >= 5; }
 
 /* Whether these products run as one launch (q8_tile.hip: more than 64 tokens, rounds on a norm more
- * than 32), and their workspace
- * is there: the library's, allocated at its first use outside a recording, or part, a caller's of
+ * than 32), and their workspace is there: the library's, allocated at its first use outside a recording, or part, a caller's of
  * Q8_GEMM_PART_MAX floats. Where not, the 64-token launches give the same bits. */
 bool tile_ready(ctx *c, int n, const long *rows, long cols, long t, bool pair, bool norm, const float *part)
 {
