@@ -235,6 +235,7 @@ struct q8_epi {
     const float *nw;
     float eps;
     const float *res;
+    int fuse = 0; /* in the product's launch on any number of rows (a recording without the workspace for apart) */
 };
 /* The decode product with the epilogue fused into its kernel (t <= 4): 0, or -1 when no fused
  * kernel takes the shape (nothing launched; the caller runs the epilogue apart). */

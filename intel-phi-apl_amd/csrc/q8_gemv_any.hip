@@ -66,7 +66,7 @@ static bool any_try(hipStream_t s, const void *w0, const void *w1, long rows, lo
     int rw = PAIR && (MT == 1 || (mid && (EPI != 1 || MT == 3))) ? 4 : 8;
     while (rw > 2 && rows / rw * nw < (PAIR ? 4096 : 1024))
         rw /= 2;
-    if (cols > 16384 || (EPI == 1 && nw > 8) || (mid && EPI && (EPI == 1 || MT == 4) && (PAIR + 1) * rows > q8_epi_rows(MT, false)))
+    if (cols > 16384 || (EPI == 1 && nw > 8) || (mid && EPI && !e.fuse && (EPI == 1 || MT == 4) && (PAIR + 1) * rows > q8_epi_rows(MT, false)))
         return false;
     if (nw <= 4)
         any_rw<MT, 4, PAIR, EPI>(s, rw, nw, w0, w1, rows, cols, x, xs, y, e);
@@ -108,7 +108,7 @@ static bool round_try(hipStream_t s, const q8_round &r, long cols, const float *
 #define ANY(N)                                                                                                         \
     Q8_LAUNCH(q8_time_name("gemv_round_any", 4, MT, Q8_ROUND_RW, N, EPI), (gemv_round_any<MT, Q8_ROUND_RW, N, EPI>), dim3((unsigned)r.start[r.n]), \
               dim3(64 * nw), s, r, cols, x, xs, e)
-    if (cols > 16384 || nw > (EPI == 1 ? 8 : MT > 2 ? 12 : 16) || (EPI == 1 && nw > 4 && r.start[r.n] * Q8_ROUND_RW > q8_epi_rows(MT, false)))
+    if (cols > 16384 || nw > (EPI == 1 ? 8 : MT > 2 ? 12 : 16) || (EPI == 1 && !e.fuse && nw > 4 && r.start[r.n] * Q8_ROUND_RW > q8_epi_rows(MT, false)))
         return false;
     if (nw <= 4)
         ANY(4);

@@ -309,7 +309,7 @@ static bool gemv_epi_go(hipStream_t s, const void *w0, const void *w1, long rows
      * round of fewer, longer workgroups) is the faster shape then (12288x4096: 20.5 against 21.3 us) */
     if (PAIR && EPI == 1 && rw == 4 && rows % 8 == 0 && rows / 8 * nw >= 2048)
         rw = 8;
-    if (EPI == 1 && kb == 8 && (PAIR + 1) * rows > q8_epi_rows(MT, PAIR))
+    if (EPI == 1 && kb == 8 && !e.fuse && (PAIR + 1) * rows > q8_epi_rows(MT, PAIR))
         return false;
     bool done = false;
     if constexpr (EPI == 2 && MT > 1)
@@ -520,7 +520,7 @@ int q8_launch_gemv_round_epi(q8_stream_t stream, int n, const void *const *w, co
     q8_round r;
     int nw;
     long kb;
-    if (!e.nw || e.res || !round_plan(n, w, rows, cols, t, y, r, nw, kb) || (kb == 8 && r.start[n] * Q8_ROUND_RW > q8_epi_rows((int)t, false)))
+    if (!e.nw || e.res || !round_plan(n, w, rows, cols, t, y, r, nw, kb) || (kb == 8 && !e.fuse && r.start[n] * Q8_ROUND_RW > q8_epi_rows((int)t, false)))
         return -1;
     hipStream_t s = (hipStream_t)stream;
     constexpr int RW = Q8_ROUND_RW;

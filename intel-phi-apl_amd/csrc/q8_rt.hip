@@ -352,10 +352,13 @@ void tile_reserve(ctx *c, int n, const long *rows, long cols, long t, bool pair,
         reserve_gemm(c, rows[0], cols, 64);
 }
 
+/* Whether the epilogue's workspace is too small for t tokens of width floats and must not grow */
+bool short_recording(ctx *c, long t, long width) { return (size_t)(t * width) > c->epi_cap && recording(c); }
+
 /* Whether a recording has to take t tokens in parts, part i of n being [t i / n, t (i + 1) / n): more than
  * 64 tokens for which the epilogue's workspace (width floats a token) is too small and must not grow. Parts
  * of more than 64 tokens hold 33 or more, so that they stay on the matrix cores and keep their bits. */
-long record_parts(ctx *c, long t, long width) { return t > 64 && (size_t)(t * width) > c->epi_cap && recording(c) ? (t + 63) / 64 : 1; }
+long record_parts(ctx *c, long t, long width) { return t > 64 && short_recording(c, t, width) ? (t + 63) / 64 : 1; }
 
 /* Whether a product of t tokens runs on the matrix cores (every 64-token launch of it, the last
  * one too, however few tokens it holds, so that a token's bits do not depend on t), else on the
@@ -539,7 +542,12 @@ void product_epi(ctx *c, const void *w0, const void *w1, long rows, long cols, c
     const bool over = overlaps(x, xs, t, cols, y, t * rows), apart = c->epi_apart != 0 || ((e.nw || t <= 4) && over);
     if (!c->exact && t <= 4 && !apart) {
         const bool timed = kt_begin(c, RT_K_GEMV + (w1 ? 1 : 0), rows, cols, t);
-        if (q8_launch_gemv_epi(s, w0, w1, rows, cols, x, xs, t, y, e) == 0) {
+        int rc = q8_launch_gemv_epi(s, w0, w1, rows, cols, x, xs, t, y, e);
+        if (rc != 0 && short_recording(c, t, e.nw ? cols : rows)) {
+            e.fuse = 1;
+            rc = q8_launch_gemv_epi(s, w0, w1, rows, cols, x, xs, t, y, e);
+        }
+        if (rc == 0) {
             launched("the product and its epilogue");
             return;
         }
@@ -1234,7 +1242,13 @@ void rt_gemv_round_norm_dev(struct rt *R, int n, const void *const *w, const lon
         for (int i = 0; i < n; i++)
             total += rows[i];
         const bool timed = kt_begin(c, RT_K_ROUND, total, cols, t);
-        if (q8_launch_gemv_round_epi(s, n, w, rows, cols, x, x_stride, t, y, q8_epi{nw, eps, nullptr}) == 0) {
+        q8_epi e{nw, eps, nullptr};
+        int rc = q8_launch_gemv_round_epi(s, n, w, rows, cols, x, x_stride, t, y, e);
+        if (rc != 0 && short_recording(c, t, cols)) {
+            e.fuse = 1;
+            rc = q8_launch_gemv_round_epi(s, n, w, rows, cols, x, x_stride, t, y, e);
+        }
+        if (rc == 0) {
             launched("the round and its norm");
             return;
         }

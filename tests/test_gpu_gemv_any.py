@@ -128,3 +128,29 @@ def test_five_to_eight_waves(rt, rows, cols, kind, t, name):
     finally:
         rt.set_epi_apart(False)
         case.close()
+
+
+@pytest.mark.parametrize("rows,cols,kind", [(4112, 8192, "norm"), (4112, 5152, "residual"), (4112, 5152, "norm"), (4112, 8192, "round_norm"), (4112, 5152, "round_norm")])
+def test_recorded_without_a_workspace(q8rt, rt, rows, cols, kind):
+    """Rows on which the epilogue runs apart, recorded by a runtime that has run nothing: fused, as it needs no
+    workspace then."""
+    case = Case(rt, rows, cols, 4, 5)
+    try:
+        case.nan()
+        case.run(kind, 0, 4)
+        want = case.out()
+    finally:
+        case.close()
+    with q8rt.Runtime() as r2:
+        c2 = Case(r2, rows, cols, 4, 5)
+        r2.lib.rt_graph_begin(r2.R)
+        c2.run(kind, 0, 4)
+        g = P(r2.lib.rt_graph_end(r2.R))
+        for _ in range(2):
+            c2.nan()
+            r2.lib.rt_graph_launch(r2.R, g)
+            for a, b in zip(c2.out(), want):
+                if not np.isnan(b).all():
+                    assert_parity(a, b.astype(np.float64), f"{kind} {rows}x{cols}")
+        r2.lib.rt_graph_free(r2.R, g)
+        c2.close()
